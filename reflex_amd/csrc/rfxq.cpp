@@ -1706,8 +1706,9 @@ int rfxq_dequantize(uint32_t ty, const void* blocks, uint64_t num_blocks, void* 
     if (reinterpret_cast<uintptr_t>(blocks) % 2u) return fail(RFXQ_ERR_OTHER, "dequantize: blocks not 2-byte aligned");
     Ctx* c;
     if (int rc = current_ctx(&c)) return rc;
-    const uint64_t groups = ty == RFXQ_TYPE_Q8_0 ? (num_blocks + 7u) / 8u : num_blocks;
-    const uint32_t grid = (uint32_t)std::min<uint64_t>(groups, 16384u);
+    // a lane per piece of 16 output bytes per run (dequant.hpp)
+    const uint64_t pieces = num_blocks * ((ty == RFXQ_TYPE_Q8_0 ? 32u : 128u) / (f16_out ? 8u : 4u));
+    const uint32_t grid = (uint32_t)std::min<uint64_t>((pieces + 255u) / 256u, 16384u);
     struct {
         const void* b;
         void* y;

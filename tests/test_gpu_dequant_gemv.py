@@ -54,6 +54,26 @@ def test_dequant_unaligned_blocks(rq, orc, ty):
     assert np.array_equal(got.view(np.uint32), orc.dequantize(ty, w, n * k).view(np.uint32))
 
 
+@pytest.mark.parametrize("ty", [Q4K, Q6K, Q8_0])
+@pytest.mark.parametrize("nb", [1, 3, 8, 517])
+def test_dequant_block_counts_and_alignment(rq, orc, ty, nb):
+    """Block counts around a workgroup's pieces; blocks 2 bytes past a 16-byte boundary and an output one element
+    past one; nothing written outside the output."""
+    qk, bb = synth.BLOCK[ty]
+    w = orc.synthetic(ty, qk * nb, 1, 31 + nb)
+    src = torch.zeros(w.size + 16, dtype=torch.uint8, device=DEV)
+    src[2:2 + w.size].copy_(_dev(w))
+    want = orc.dequantize(ty, w, nb * qk)
+    for dt, ref in ((torch.float32, want), (torch.float16, want.astype(np.float16))):
+        out = torch.full((nb * qk + 10,), 7.0, dtype=dt, device=DEV)
+        rc = rq.lib().rfxq_dequantize(ty, src.data_ptr() + 2, nb, out.data_ptr() + out.element_size(),
+                                      int(dt == torch.float16), torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        got = out.cpu().numpy()
+        assert got[1:1 + nb * qk].tobytes() == ref.tobytes()
+        assert got[0] == 7.0 and (got[1 + nb * qk:] == 7.0).all()
+
+
 def test_dequant_committed_fixtures(rq):
     import os
     f = np.load(os.path.join(os.path.dirname(__file__), "golden", "fixtures.npz"))
