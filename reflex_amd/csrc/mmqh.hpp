@@ -126,36 +126,42 @@ RFXQ_DEV uint32_t act_chunk(uint32_t tid) { return (tid & 7u) ^ ((tid >> 4) & 7u
 RFXQ_DEV uint32_t f16_rne(float v) { return __builtin_bit_cast(uint16_t, (half_t)v); }
 RFXQ_DEV uint32_t pack16(uint32_t lo, uint32_t hi) { return (lo & 0xFFFFu) | (hi << 16); }
 
-// the 6-bit scales and mins of sub-blocks 0..7 (get_scale_min_k4,
-// src/dequant.rs:39-47) from header dwords y, z, w (bytes 4..15)
-RFXQ_DEV void q4k_scales_mins(const u4_t hdr, float (&sc)[8], float (&mn)[8]) {
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        sc[j] = (float)((hdr.y >> (8 * j)) & 63u);
-        mn[j] = (float)((hdr.z >> (8 * j)) & 63u);
-        sc[j + 4] = (float)(((hdr.w >> (8 * j)) & 0xFu) | (((hdr.y >> (8 * j + 6)) & 3u) << 4));
-        mn[j + 4] = (float)(((hdr.w >> (8 * j + 4)) & 0xFu) | (((hdr.z >> (8 * j + 6)) & 3u) << 4));
-    }
-}
-
-// Per super-block operands of one weight column: the constant-part A operand
-// (C_0..7 as f16 pairs) and the eight block multipliers, packed two per dword
-// (block 2p low, 2p + 1 high): f16(d*sc_b) for the low-nibble blocks (even
-// b), f16(d*sc_b/16) for the high-nibble ones (the codes' scales 1 and 16).
+// Per super-block operands of one weight column from its header (all lanes of
+// both halves hold it): the constant-part A operand (C_0..7 as f16 pairs) and
+// the eight block multipliers, packed two per dword (block 2p low, 2p + 1
+// high): f16(d*sc_b) for the low-nibble blocks (even b), f16(d*sc_b/16) for
+// the high-nibble ones (the codes' scales 1 and 16). The 6-bit scales and
+// mins (get_scale_min_k4, src/dequant.rs:39-47) stay four to a dword: for the
+// multipliers a byte pair goes into the mantissas of two f16 1024.0, an exact
+// fma leaves (sc, sc/16) and one multiply rounds. The constants take f32
+// arithmetic, four blocks in each lane half, exchanged at the end (54 VALU
+// instructions a header against 90 for one block at a time in both halves).
 RFXQ_DEV void q4k_sb_operands(const u4_t hdr, u4_t& cop, u4_t& dsc) {
-    float sc[8], mn[8];
-    q4k_scales_mins(hdr, sc, mn);
-    const float d = f16_bits_to_f32(hdr.x), dmin = f16_bits_to_f32(hdr.x >> 16);
-    uint32_t c[8], s[8];
-#pragma unroll
-    for (int b = 0; b < 8; b++) {
-        c[b] = f16_rne(__builtin_fmaf(8.0f * d, sc[b], -(dmin * mn[b])));
-        s[b] = f16_rne(d * sc[b] * ((b & 1) ? 0.0625f : 1.0f));
-    }
+    const uint32_t sc_lo = hdr.y & 0x3F3F3F3Fu, mn_lo = hdr.z & 0x3F3F3F3Fu;
+    const uint32_t sc_hi = (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u);
+    const uint32_t mn_hi = ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u);
+    const uint32_t dd = __builtin_amdgcn_perm(hdr.x, hdr.x, 0x01000100u);
+    const h2_t scale = {(half_t)1.0f, (half_t)0.0625f}, off = {(half_t)-1024.0f, (half_t)-64.0f};
 #pragma unroll
     for (int p = 0; p < 4; p++) {
-        cop[p] = pack16(c[2 * p], c[2 * p + 1]);
-        dsc[p] = pack16(s[2 * p], s[2 * p + 1]);
+        const uint32_t b = __builtin_amdgcn_perm(0x64646464u, p < 2 ? sc_lo : sc_hi, (p & 1) ? 0x04030402u : 0x04010400u);
+        h2_t v = __builtin_elementwise_fma(as_h2(b), scale, off);
+        asm("" : "+v"(v));  // exact; the product below rounds
+        dsc[p] = h2_bits(v * as_h2(dd));
+    }
+    const bool up = (threadIdx.x & 32u) != 0u;
+    const uint32_t sc = up ? sc_hi : sc_lo, mn = up ? mn_hi : mn_lo;
+    const float d8 = 8.0f * f16_bits_to_f32(hdr.x), dmin = f16_bits_to_f32(hdr.x >> 16);
+    uint32_t c[4];
+#pragma unroll
+    for (int b = 0; b < 4; b++)
+        c[b] = f16_rne(__builtin_fmaf(d8, (float)((sc >> (8 * b)) & 0xFFu), -(dmin * (float)((mn >> (8 * b)) & 0xFFu))));
+#pragma unroll
+    for (int p = 0; p < 2; p++) {
+        const uint32_t v = pack16(c[2 * p], c[2 * p + 1]);
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        cop[p] = r[0];
+        cop[2 + p] = r[1];
     }
 }
 
