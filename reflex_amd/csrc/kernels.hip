@@ -9,5 +9,6 @@
 #include "quant.hpp"
 #include "mmq.hpp"
 #include "mmqh.hpp"
+#include "mmqs.hpp"
 #include "moe.hpp"
 #include "moe_decode.hpp"

@@ -152,6 +152,7 @@ struct Ctx {
     hipFunction_t mmq[3] = {}, dots[3] = {}, mmq64[3] = {};
     hipFunction_t mmqh[3][3] = {};  // [Q4_K, Q6_K, Q8_0][128-row, 32-row, 64-row tiles]
     hipFunction_t mmqh_mix_m32 = nullptr;  // 32-row tiles, Q4_K or Q6_K per descriptor
+    hipFunction_t mmqs = nullptr;          // up to 32 rows, any type per descriptor
     hipFunction_t act_f16 = nullptr, act_f16_multi = nullptr, act_f16_wg = nullptr, act_f16_multi_wg = nullptr;
     hipFunction_t deq[3][2] = {};
     hipFunction_t gather = nullptr, scatter = nullptr, silu = nullptr, combine = nullptr;
@@ -229,6 +230,7 @@ int load_ctx(int device, Ctx** out) {
         {&c->mmqh[2][1], "rfxq_mmqh_q8_0_m32"},
         {&c->mmqh[2][2], "rfxq_mmqh_q8_0_m64"},
         {&c->mmqh_mix_m32, "rfxq_mmqh_mix_m32"},
+        {&c->mmqs, "rfxq_mmqs"},
         {&c->act_f16, "rfxq_act_f16"},
         {&c->act_f16_multi, "rfxq_act_f16_multi"},
         {&c->act_f16_wg, "rfxq_act_f16_wg"},
@@ -900,6 +902,14 @@ uint32_t split_sb(const std::vector<std::pair<uint32_t, uint32_t>>& tiles_nsb, u
 // above
 uint32_t f16_tile_m(uint32_t rows) { return rows <= 32u ? 32u : rows <= 64u ? 64u : kMmqBM; }
 
+// Super-blocks that one workgroup of the few-row kernel (mmqs.hpp) can hold
+// the activations of (16 rows of 8, 32 rows of 4: its staging registers, and
+// 70 KB of LDS so that two workgroups fit a CU); 0 above its 32 rows.
+uint32_t few_max_sb(uint32_t rows) { return rows > 32u ? 0u : rows > 16u ? 4u : 8u; }
+uint32_t few_lds(uint32_t rows, uint32_t sb) {
+    return 128u + std::max(16384u, rows * (sb * 544u + 16u));  // (results pass through 4 KB per wave)
+}
+
 // Row tile of one grouped MoE GEMM, `pairs` routed rows over `experts`
 // groups, `tiles_n` column tiles per expert: f16 kernels 32-row tiles up to
 // 12 rows per expert on average, 128 above 64; in between 64 or 128,
@@ -972,10 +982,13 @@ rfxq_gemm_policy gemm_policy(uint32_t ty, uint32_t k, uint32_t n, uint32_t rows,
     if (f16 && alone && !o.quant_mma_splits && rows >= 256u) p.tile_m = small_gemm_tile_m(p.tile_m, rows, n, nsb, cus);
     const uint32_t tiles = ((rows + p.tile_m - 1u) / p.tile_m) * ((n + p.tile_n - 1u) / p.tile_n);
     uint32_t splits = 1;
+    const uint32_t few = f16 ? few_max_sb(rows) : 0u;
     if (o.quant_mma_splits) splits = o.quant_mma_splits;
-    else if (2u * tiles < std::max(cus, 1u)) {
-        // 32-row tiles stream weights (few rows): splits down to one super-block
-        const uint32_t w = split_sb({{tiles, nsb}}, p.tile_m == 32u ? 1u : 2u, 2u * std::max(cus, 1u));
+    else if (2u * tiles < std::max(cus, 1u) || few) {
+        // 32-row tiles stream weights (few rows): splits down to one
+        // super-block, and ranges that the few-row kernel can hold
+        uint32_t w = split_sb({{tiles, nsb}}, p.tile_m == 32u ? 1u : 2u, 2u * std::max(cus, 1u));
+        if (few) w = std::min(w, few);
         splits = (nsb + w - 1u) / w;
     }
     splits = std::min(std::max(1u, splits), nsb);
@@ -1160,6 +1173,33 @@ int launch_mmq(Ctx* c, uint32_t ty, const MmqDesc* descs, uint32_t count, const 
     return launch(f, total_wgs, 0, stream, &a, sizeof a, "rfxq_mmq launch", kMmqThreads);
 }
 
+// rfxq_mmqs over descriptors of at most 32 rows (one row tile each)
+int launch_few(Ctx* c, const MmqDesc* descs, uint32_t count, const MmqDesc* table, uint32_t total_wgs,
+               hipStream_t stream) {
+    MmqArgs a;
+    std::memset(&a, 0, sizeof a);
+    a.ndesc = count;
+    a.table = table;
+    if (count <= kMmqInline) std::copy(descs, descs + count, a.inl);
+    uint32_t lds = 0;
+    for (uint32_t i = 0; i < count; i++) lds = std::max(lds, few_lds(descs[i].m, descs[i].sb_per_split));
+    return launch(c->mmqs, total_wgs, lds, stream, &a, sizeof a, "rfxq_mmqs launch", kMmqThreads);
+}
+
+// [a, a + na) and [b, b + nb) share bytes
+bool overlap(const void* a, uint64_t na, const void* b, uint64_t nb) {
+    const uintptr_t pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
+    return pa < pb + nb && pb < pa + na;
+}
+
+// the descriptor fields of an rfxq_mmqs GEMM reading f32 rows
+void few_act_desc(MmqDesc* d, const float* x) {
+    d->xq = reinterpret_cast<const int8_t*>(x);
+    d->xds = nullptr;
+    d->xrs = nullptr;
+    d->ldq = 4u * d->k;
+}
+
 int check_mmq_weight(const rfxq_weight* w, const char* what) {
     if (int rc = check_weight(w, what)) return rc;
     if (w->in_features % 256u)
@@ -1171,13 +1211,15 @@ int check_mmq_weight(const rfxq_weight* w, const char* what) {
 struct GemmPlan {
     rfxq_gemm_policy pol;
     bool f16 = false;
+    bool few = false;  // on rfxq_mmqs (which reads f32 activations: no layout)
     uint32_t tiles_m = 1, tiles_n = 1;
     ActLayout act;
     uint64_t off_part = 0, total = 0;
 };
 
 // an MMQ plan for a GEMM the policy sends to an MMQ path
-GemmPlan plan_gemm(const Ctx* c, const rfxq_weight* w, uint32_t rows, const rfxq_options& o) {
+// (`in_place`: y overlaps x, which must then be read before any result is written)
+GemmPlan plan_gemm(const Ctx* c, const rfxq_weight* w, uint32_t rows, const rfxq_options& o, bool in_place = false) {
     GemmPlan p;
     const uint32_t k = w->in_features, n = w->out_features;
     p.pol = gemm_policy(w->ggml_type, k, n, rows, c ? (uint32_t)c->cus : 256u, o);
@@ -1185,7 +1227,8 @@ GemmPlan plan_gemm(const Ctx* c, const rfxq_weight* w, uint32_t rows, const rfxq
     if (p.pol.path == PATH_GEMV_ROWS) return p;  // no MMQ launch: tiles, layouts and workspace stay 0
     p.tiles_m = (rows + p.pol.tile_m - 1u) / p.pol.tile_m;
     p.tiles_n = (n + p.pol.tile_n - 1u) / p.pol.tile_n;
-    p.act = act_layout_sel(rows, k, !p.f16, p.f16);
+    p.few = p.f16 && !in_place && p.pol.sb_per_split <= few_max_sb(rows);
+    if (!p.few) p.act = act_layout_sel(rows, k, !p.f16, p.f16);
     p.off_part = p.act.total;
     p.total = p.off_part + (p.pol.splits > 1 ? align256((uint64_t)p.pol.splits * rows * n * 4u) : 0u);
     return p;
@@ -1202,19 +1245,21 @@ int launch_reduce(Ctx* c, const float* part, float* y, uint64_t n, uint32_t spli
     return launch(c->reduce, (uint32_t)blocks, 0, stream, &a, sizeof a, "rfxq_splitk_reduce launch");
 }
 
-// One GEMM's MMQ launch from activation layouts (`act`, layouts p.act), then
-// the split-K reduce when p splits K (partials in `part`).
-int gemm_run(Ctx* c, const GemmPlan& p, const uint8_t* act, const ActLayout& L, const rfxq_weight* w,
+// One GEMM's MMQ launch from activation layouts (`act`, layouts L) or, for the
+// few-row kernel, f32 rows `x` (else NULL), then the split-K reduce when p
+// splits K (partials in `part`).
+int gemm_run(Ctx* c, const GemmPlan& p, const float* x, const uint8_t* act, const ActLayout& L, const rfxq_weight* w,
              uint32_t rows, float* y, float* part, hipStream_t stream) {
     const uint32_t k = w->in_features, n = w->out_features;
     MmqDesc d;
     std::memset(&d, 0, sizeof d);
     d.w = w->data;
-    act_desc(&d, act, L, p.f16, k);
+    d.k = k;
+    if (x) few_act_desc(&d, x);
+    else act_desc(&d, act, L, p.f16, k);
     d.y = p.pol.splits > 1 ? part : y;
     d.m = rows;
     d.n = n;
-    d.k = k;
     d.type = w->ggml_type;
     d.ldy = n;
     d.tiles_m = p.tiles_m;
@@ -1222,7 +1267,8 @@ int gemm_run(Ctx* c, const GemmPlan& p, const uint8_t* act, const ActLayout& L, 
     d.splits = p.pol.splits;
     d.sb_per_split = p.pol.sb_per_split;
     const uint32_t wgs = p.tiles_m * p.tiles_n * p.pol.splits;
-    if (int rc = launch_mmq(c, w->ggml_type, &d, 1, nullptr, wgs, false, stream, p.f16, p.pol.tile_m))
+    if (int rc = p.few ? launch_few(c, &d, 1, nullptr, wgs, stream)
+                       : launch_mmq(c, w->ggml_type, &d, 1, nullptr, wgs, false, stream, p.f16, p.pol.tile_m))
         return rc;
     if (p.pol.splits > 1)
         if (int rc = launch_reduce(c, part, y, (uint64_t)rows * n, p.pol.splits, stream)) return rc;
@@ -1231,7 +1277,8 @@ int gemm_run(Ctx* c, const GemmPlan& p, const uint8_t* act, const ActLayout& L, 
 
 int gemm_impl(Ctx* c, const float* x, const rfxq_weight* w, uint32_t rows, float* y, void* ws, uint64_t ws_bytes,
               const rfxq_options& o, hipStream_t stream) {
-    const GemmPlan p = plan_gemm(c, w, rows, o);
+    const bool in_place = overlap(x, 4ull * rows * w->in_features, y, 4ull * rows * w->out_features);
+    const GemmPlan p = plan_gemm(c, w, rows, o, in_place);
     if (!ws) {
         if (int rc = ctx_workspace(c, p.total, &ws, stream)) return rc;
     } else if (ws_bytes < p.total) {
@@ -1239,8 +1286,9 @@ int gemm_impl(Ctx* c, const float* x, const rfxq_weight* w, uint32_t rows, float
                     (unsigned long long)ws_bytes, (unsigned long long)p.total);
     }
     uint8_t* base = static_cast<uint8_t*>(ws);
-    if (int rc = launch_act(c, x, rows, w->in_features, base, p.act, !p.f16, p.f16, stream)) return rc;
-    return gemm_run(c, p, base, p.act, w, rows, y, reinterpret_cast<float*>(base + p.off_part), stream);
+    if (!p.few)
+        if (int rc = launch_act(c, x, rows, w->in_features, base, p.act, !p.f16, p.f16, stream)) return rc;
+    return gemm_run(c, p, p.few ? x : nullptr, base, p.act, w, rows, y, reinterpret_cast<float*>(base + p.off_part), stream);
 }
 
 int check_act(const void* act, uint32_t rows, uint32_t k, const char* what) {
@@ -1259,8 +1307,8 @@ int check_act(const void* act, uint32_t rows, uint32_t k, const char* what) {
 // takes the single-GEMM policy's path (gemm_policy); GEMMs on the GEMV path
 // run as one GEMV per row in one table-driven launch.
 // type_index + 3 * variant (0: int8, 1: int8 64-row, 2: f16, 3: f16 32-row,
-// 4: f16 64-row)
-constexpr uint32_t kGroupKernels = 15;
+// 4: f16 64-row); last the few-row kernel, every type
+constexpr uint32_t kGroupFew = 15, kGroupKernels = 16;
 struct GemmGroup {
     struct Act {
         const float* x;
@@ -1293,7 +1341,7 @@ struct GemmGroup {
 bool group_f16(uint32_t g) { return g >= 6u; }
 uint32_t group_tile_m(uint32_t g) {
     const uint32_t v = g / 3u;
-    return v == 1u || v == 4u ? 64u : v == 3u ? 32u : kMmqBM;
+    return v == 1u || v == 4u ? 64u : v == 3u || v == 5u ? 32u : kMmqBM;
 }
 uint32_t group_variant(bool f16, uint32_t tile_m) { return f16 ? (tile_m == 32u ? 3u : tile_m == 64u ? 4u : 2u) : (tile_m == 64u ? 1u : 0u); }
 // the group (launch) of a GEMM: type_index + 3 * variant, except that the f16
@@ -1314,6 +1362,13 @@ int build_gemm_group(const rfxq_gemm_item* items, uint32_t count, uint32_t rows,
     uint64_t group_bytes = 0;  // the few-row path is chosen for the group as a whole
     for (uint32_t i = 0; i < count; i++)
         if (items[i].w) group_bytes += gemm_weight_bytes(items[i].w->ggml_type, items[i].w->in_features, items[i].w->out_features);
+    // the few-row kernel reads f32 activations while results are written: not
+    // for a group with an output on one of its inputs
+    bool in_place = false;
+    for (uint32_t i = 0; i < count && few_max_sb(rows) && !ext; i++)
+        for (uint32_t j = 0; j < count && items[i].w; j++)
+            in_place |= items[j].w && overlap(items[i].x, 4ull * rows * items[i].w->in_features, items[j].y,
+                                              4ull * rows * items[j].w->out_features);
     for (uint32_t i = 0; i < count; i++) {
         const rfxq_gemm_item& it = items[i];
         if (int rc = check_weight(it.w, "gemm group")) return rc;
@@ -1336,7 +1391,9 @@ int build_gemm_group(const rfxq_gemm_item* items, uint32_t count, uint32_t rows,
             continue;
         }
         const bool f16 = pol.path == PATH_MMQ_F16;
-        item_kernel[i] = group_index(it.w->ggml_type, f16, pol.tile_m);
+        const uint32_t nsb = k / 256u, ns = std::min(o.quant_mma_splits, nsb);  // a forced split may leave too long ranges
+        const bool few = f16 && !in_place && few_max_sb(rows) && (!ns || (nsb + ns - 1u) / ns <= few_max_sb(rows));
+        item_kernel[i] = few ? kGroupFew : group_index(it.w->ggml_type, f16, pol.tile_m);
         size_t ai = 0;
         while (ai < g->acts.size() && g->acts[ai].x != it.x) ai++;
         if (ai == g->acts.size()) {
@@ -1349,7 +1406,7 @@ int build_gemm_group(const rfxq_gemm_item* items, uint32_t count, uint32_t rows,
             return fail(RFXQ_ERR_OTHER, "gemm group: one x used with in_features %u and %u", g->acts[ai].k, k);
         }
         item_act[i] = (uint32_t)ai;
-        if (f16) g->acts[ai].need_h = true;
+        if (f16) g->acts[ai].need_h |= !few;
         else g->acts[ai].need_i8 = true;
     }
     for (auto& a : g->acts) {
@@ -1393,12 +1450,13 @@ int build_gemm_group(const rfxq_gemm_item* items, uint32_t count, uint32_t rows,
     bool split_small[kGroupKernels] = {};
     for (uint32_t t = 0; t < kGroupKernels; t++) {
         auto& v = g->descs[t];
-        if (v.empty() || (!forced && 2u * g->wgs[t] >= cus)) continue;
+        if (v.empty() || (!forced && 2u * g->wgs[t] >= cus && t != kGroupFew)) continue;
         split_small[t] = true;
         // one split size for the launch, so its workgroups take alike
         std::vector<std::pair<uint32_t, uint32_t>> tn;
         for (const auto& d : v) tn.push_back({d.tiles_m * d.tiles_n, d.k / 256u});
-        const uint32_t w_sb = split_sb(tn, group_tile_m(t) == 32u ? 1u : 2u, 2u * std::max(cus, 1u));
+        uint32_t w_sb = split_sb(tn, group_tile_m(t) == 32u ? 1u : 2u, 2u * std::max(cus, 1u));
+        if (t == kGroupFew) w_sb = std::min(w_sb, few_max_sb(rows));
         uint32_t wg = 0;
         for (uint32_t i = 0; i < v.size(); i++) {
             MmqDesc& d = v[i];
@@ -1483,6 +1541,7 @@ int build_gemm_group(const rfxq_gemm_item* items, uint32_t count, uint32_t rows,
 int launch_group_kernel(Ctx* c, const GemmGroup& g, uint32_t t, const MmqDesc* table, hipStream_t stream) {
     const auto& v = g.descs[t];
     if (v.empty()) return RFXQ_OK;
+    if (t == kGroupFew) return launch_few(c, v.data(), (uint32_t)v.size(), table, g.wgs[t], stream);
     return launch_mmq(c, v[0].type, v.data(), (uint32_t)v.size(), table, g.wgs[t], false, stream, group_f16(t),
                       group_tile_m(t));
 }
@@ -1517,7 +1576,8 @@ void bind_gemm_group(GemmGroup* g, uint8_t* ws) {
         for (size_t i = 0; i < g->descs[t].size(); i++) {
             MmqDesc& d = g->descs[t][i];
             const GemmGroup::Act& a = g->acts[g->act_of[t][i]];
-            act_desc(&d, a.base(ws), a.L, group_f16(t), d.k);
+            if (t == kGroupFew && !a.ext) few_act_desc(&d, a.x);
+            else act_desc(&d, a.base(ws), a.L, group_f16(t), d.k);
         }
     for (auto& r : g->reduces) {
         r.part = reinterpret_cast<float*>(ws + r.off);
@@ -1976,7 +2036,9 @@ int rfxq_gemm_batch(const rfxq_gemm_item* items, uint32_t count, uint32_t rows, 
                 d[j].wg_begin = wg;
                 wg += d[j].tiles_m * d[j].tiles_n * d[j].splits;
             }
-            if (int rc = launch_mmq(c, d[0].type, d, cnt, nullptr, wg, false, stream, group_f16(t), group_tile_m(t)))
+            if (int rc = t == kGroupFew ? launch_few(c, d, cnt, nullptr, wg, stream)
+                                        : launch_mmq(c, d[0].type, d, cnt, nullptr, wg, false, stream, group_f16(t),
+                                                     group_tile_m(t)))
                 return rc;
         }
         if (int rc = run_group_reduces(c, g, t, stream)) return rc;
@@ -2090,7 +2152,7 @@ int rfxq_gemm_q8_1(const void* act, uint32_t rows, const rfxq_weight* w, float* 
         }
         part = static_cast<float*>(ws);
     }
-    if (int rc = gemm_run(c, p, static_cast<const uint8_t*>(act), act_layout(rows, k), w, rows, y, part, stream))
+    if (int rc = gemm_run(c, p, nullptr, static_cast<const uint8_t*>(act), act_layout(rows, k), w, rows, y, part, stream))
         return rc;
     return ok();
 }

@@ -307,6 +307,28 @@ def test_gemm_weight_past_4gib(rq, orc, ty):
     assert e < TOL
 
 
+@pytest.mark.parametrize("ty", [Q4K, Q6K, Q8_0])
+@pytest.mark.parametrize("m,n,k", [(5, 70, 256), (16, 257, 2304), (17, 255, 1280), (32, 600, 4864), (9, 513, 14336)])
+def test_gemm_few_rows_kernel(rq, orc, ty, m, n, k):
+    """The few-row kernel at its edges: ragged column tiles, ranges of 1 to 8 super-blocks (16 rows)
+    and of 4 (17 rows up), a short last range; weights 2 bytes past a dword; an activation buffer instead of f32
+    rows; and an output over its own input, which takes the tile kernels."""
+    w_np = synth.weights(ty, n, k, 900 + m)
+    x_np = synth.activations(m * k, 901 + m).reshape(m, k)
+    y, _ = _check_gemm(rq, orc, ty, m, n, k, w_np, x_np)
+    x, w = _dev(x_np.reshape(-1)), _weight(rq, ty, w_np, n, k)
+    assert np.array_equal(rq.gemm_q8_1(rq.quantize_act_q8_1(x, m, k), w, m).cpu().numpy().reshape(m, n), y)
+    if ty != Q4K:
+        buf = torch.zeros(w_np.size + 16, dtype=torch.uint8, device=DEV)
+        buf[2:2 + w_np.size] = _dev(w_np)
+        w2 = rq.Weight(rq.GgmlType(ty), buf, [k, n], offset=2, len=w_np.size)
+        assert np.array_equal(rq.gemm(x, w2, m).cpu().numpy().reshape(m, n), y)
+    if n <= k:
+        over = x.clone()
+        got = rq.gemm(over, w, m, out=over)[:m * n].cpu().numpy().reshape(m, n)
+        assert np.abs(got - y).max() <= 1e-5 * np.abs(y).max()
+
+
 def test_gemm_rows_independent_and_deterministic(rq, orc, opts):
     """Row r of the output depends only on row r of x, and repeats give identical bits."""
     n, k = 1024, 2048
