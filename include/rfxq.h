@@ -110,7 +110,11 @@ int rfxq_set_options(const rfxq_options* options);
  * (splits ranges of sb_per_split super-blocks); tile and splits are 0/1 on the
  * GEMV path. Counterpart of quant_mma_splits / quant_mma_block_rows /
  * quant_mma_max_rows (kernels.rs:628-713) and the fused-GEMV crossover
- * (:2144-2169), re-derived for MI355X; `compute_units` as the device reports. */
+ * (:2144-2169), re-derived for MI355X; `compute_units` as the device reports.
+ * tile and splits are the general plan's. Unless REFLEX_QUANT_MMA_SPLITS
+ * forces a count, a GEMM of more than 32 rows may run on 64 x 128 tiles with
+ * fewer ranges instead, where that is estimated faster; the sum over K is then
+ * cut at other places. */
 typedef struct rfxq_gemm_policy {
     uint32_t path;
     uint32_t tile_m, tile_n;

@@ -210,6 +210,13 @@ RFXQ_DEV uint32_t act_row(const MmqDesc& ds, uint32_t r) {
 // (the host keeps those activations under 4 GiB).
 RFXQ_DEV uint32_t act_base(const MmqDesc& ds, uint32_t m0) { return ds.rows ? 0u : m0; }
 
+// The scale 2^e of the tile's row tid (for the stores): read before the loop,
+// written to LDS after it; a buffer load, so no wait before the first stage
+// covers it.
+RFXQ_DEV float row_scale_load(const MmqDesc& ds, uint32_t m0, uint32_t tid, uint32_t bm) {
+    return tid < bm && m0 + tid < ds.m ? as_f32(bld4(make_rsrc(ds.xrs, 0xFFFFFFFFu), 4u * act_row(ds, m0 + tid))) : 0.0f;
+}
+
 // The accumulator of a 32x32 output tile (mfma16: A = activations, B =
 // weights): lane (l32, h) holds weight column l32 and activation rows
 // 8 q4 + 4 h + r (q4, r in [0, 4)) as acc[4 q4 + r]. Stored as dwords: the
@@ -233,7 +240,7 @@ RFXQ_DEV void store_tile(const MmqDesc& ds, float* y, uint32_t row, uint32_t col
     }
 }
 
-// A wave's MT x 2 accumulator tiles (rows m0 + 32i, columns c0 + 32j) with
+// A wave's MT x NJ accumulator tiles (rows m0 + 32i, columns c0 + 32j) with
 // 16-byte stores: each tile passes through the wave's 4 KB LDS region `buf`
 // (free once the tile loop is over) as a row-major 32x32 array whose column
 // index is xor'ed with 4 (R % 8) in row R (whole float4 groups stay
@@ -241,15 +248,15 @@ RFXQ_DEV void store_tile(const MmqDesc& ds, float* y, uint32_t row, uint32_t col
 // columns 4k..4k+3: eight lanes per 128-byte row piece and a quarter of the
 // dword stores' instructions (4-5% of the 0.6B prefill set). Outputs whose
 // rows are not 16-byte aligned take the dword stores.
-template <int MT, int JMASK = 3>
-RFXQ_DEV void store_wave(const MmqDesc& ds, float* y, uint32_t m0, uint32_t c0, const v16f_t (&acc)[MT][2],
+template <int MT, int NJ, int JMASK = 3>
+RFXQ_DEV void store_wave(const MmqDesc& ds, float* y, uint32_t m0, uint32_t c0, const v16f_t (&acc)[MT][NJ],
                          const float* sc, u4_t* buf, bool scale = true) {
     const uint32_t lane = threadIdx.x & 63u, l32 = lane & 31u, h = lane >> 5;
     if ((ds.ldy & 3u) != 0u || (reinterpret_cast<uintptr_t>(y) & 15u) != 0u) {
 #pragma unroll
         for (int i = 0; i < MT; i++)
 #pragma unroll
-            for (int j = 0; j < 2; j++)
+            for (int j = 0; j < NJ; j++)
                 if (JMASK >> j & 1)
                     store_tile(ds, y, m0 + 32u * i + 4u * h, c0 + 32u * j + l32, acc[i][j], sc + 32u * i + 4u * h, scale);
         return;
@@ -259,7 +266,7 @@ RFXQ_DEV void store_wave(const MmqDesc& ds, float* y, uint32_t m0, uint32_t c0, 
 #pragma unroll
     for (int i = 0; i < MT; i++)
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
+        for (int j = 0; j < NJ; j++) {
             if (!(JMASK >> j & 1)) continue;
 #pragma unroll
             for (int q4 = 0; q4 < 4; q4++)
@@ -373,20 +380,20 @@ RFXQ_DEV u4_t q6k_multipliers(u4_t sc, uint32_t dbits, uint32_t h) {
 }  // namespace mmqh
 
 
-// One (32 MT)x256 tile (and one split-K range) of Y = X . W^T for Q4_K weights.
-template <int MT>
-RFXQ_DEV void mmqh_q4k_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_t ks, const mmqh::ActLds& L) {
+// Accumulators of one (32 MT) x (128 NJ) tile of Y = X . W^T over super-blocks
+// [sb0, sb1) for Q4_K weights.
+template <int MT, int NJ>
+RFXQ_DEV void mmqh_q4k_acc(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_t sb0, uint32_t sb1,
+                           const mmqh::ActLds& L, v16f_t (&acc)[MT][NJ], float& row_scale) {
     using namespace mmqh;
     constexpr uint32_t BM = Tile<MT>::BM;
-    // weight loads per stage: the code pieces of two stages (four loads) at
+    // weight loads per stage: the code pieces of two stages (two loads a column tile) at
     // even positions, with the headers at position 0; none at odd ones
     constexpr int WA = 2;
-    using Pipe = StagePipe<MT, WA, 6, 0, 4, 0, 1>;
+    using Pipe = StagePipe<MT, WA, 3 * NJ, 0, 2 * NJ, 0, 1>;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, l32 = lane & 31u, h = lane >> 5;
     const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t nsb = ds.k / 256u;
-    const uint32_t sb0 = ks * ds.sb_per_split;
-    const uint32_t sb1 = min(nsb, sb0 + ds.sb_per_split);
     const uint32_t row_bytes = nsb * 144u;
     const uint32_t rec_bytes = nsb * 32u;
 
@@ -397,11 +404,11 @@ RFXQ_DEV void mmqh_q4k_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_
     const rsrc_t r_act = make_rsrc(ds.xq + (uint64_t)rb * ds.ldq, 0xFFFFFFFFu);
     // a gate/up pair: waves 0-1 the gate columns [n0, n0 + 128), waves 2-3
     // the same columns of up
-    const bool pair = ds.gu_pair != 0u;
+    const bool pair = NJ == 2 && ds.gu_pair != 0u;
     const bool upw = pair && w >= 2u;
     const uint32_t wc = pair ? (w & 1u) : w;  // the wave's 64-column block
     const rsrc_t r_w = make_rsrc((upw ? ds.w_up : ds.w) + (uint64_t)n0 * row_bytes,
-                                 min(pair ? BN / 2u : BN, ds.n - n0) * row_bytes);
+                                 min(pair ? BN / 2u : 128u * NJ, ds.n - n0) * row_bytes);
     const rsrc_t r_sx =
         make_rsrc(reinterpret_cast<const uint8_t*>(ds.xds) + (uint64_t)rb * rec_bytes, 0xFFFFFFFFu);
     // Staged activations, copied straight into LDS (buffer_load ... lds: the
@@ -426,12 +433,12 @@ RFXQ_DEV void mmqh_q4k_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_
     // quant bytes of column 64w + 32j + l32 for each stage. Each lane also
     // loads its column's 16-byte header with the first stage of each
     // super-block.
-    uint32_t col[2], g_q[2], g_h[2];
+    uint32_t col[NJ], g_q[NJ], g_h[NJ];
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        col[j] = 64u * wc + 32u * j + l32;
+    for (int j = 0; j < NJ; j++) {
+        col[j] = 32u * NJ * wc + 32u * j + l32;
         g_h[j] = col[j] * row_bytes;
-        g_q[j] = (64u * wc + 32u * j + (l32 & 15u)) * row_bytes + 16u + 32u * (l32 >> 4) + 16u * h;
+        g_q[j] = (32u * NJ * wc + 32u * j + (l32 & 15u)) * row_bytes + 16u + 32u * (l32 >> 4) + 16u * h;
     }
     const uint32_t g_qb = 16u * row_bytes;  // load B: 16 columns on
     const uint32_t nst = 4u * (sb1 - sb0);
@@ -452,23 +459,22 @@ RFXQ_DEV void mmqh_q4k_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_
     };
     // weights of two stage pairs (by pair: loads A, B of each n-tile), a
     // super-block's headers; load_w takes an even stage st: stages st, st + 1
-    u4_t qp[2][2][2], hn[2];
+    u4_t qp[2][NJ][2], hn[NJ];
     auto load_w = [&](uint32_t st, bool hdr) {
         const uint32_t sl = min(st, nst - 2u);
         const uint32_t sb = sb0 + (sl >> 2), g = sl & 3u;
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
+        for (int j = 0; j < NJ; j++) {
             qp[(st >> 1) & 1u][j][0] = __builtin_amdgcn_raw_buffer_load_b128(r_w, g_q[j], 144u * sb + 32u * g, 0);
             qp[(st >> 1) & 1u][j][1] = __builtin_amdgcn_raw_buffer_load_b128(r_w, g_q[j] + g_qb, 144u * sb + 32u * g, 0);
         }
         if (hdr)
 #pragma unroll
-            for (int j = 0; j < 2; j++) hn[j] = __builtin_amdgcn_raw_buffer_load_b128(r_w, g_h[j], 144u * sb, 0);
+            for (int j = 0; j < NJ; j++) hn[j] = __builtin_amdgcn_raw_buffer_load_b128(r_w, g_h[j], 144u * sb, 0);
     };
 
-    v16f_t acc[MT][2];
 #pragma unroll
-    for (int i = 0; i < MT; i++) acc[i][0] = acc[i][1] = v16f_t{};
+    for (int i = 0; i < MT; i++) for (int j = 0; j < NJ; j++) acc[i][j] = v16f_t{};
     // LDS read offsets (16-byte units): activations of row l32 of row tile 0,
     // logical chunk 4e + 2h + step
     uint32_t a_act[2][2];
@@ -476,30 +482,26 @@ RFXQ_DEV void mmqh_q4k_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_
     for (int e = 0; e < 2; e++)
 #pragma unroll
         for (int s2 = 0; s2 < 2; s2++) a_act[e][s2] = l32 * 8u + ((4u * e + 2u * h + s2) ^ ((l32 >> 1) & 7u));
-    u4_t dsc[2] = {}, q[2] = {};
+    u4_t dsc[NJ] = {}, q[NJ] = {};
     // code-extraction constants, kept in VGPRs (VOP3 takes no literal here)
     uint32_t mlo = 0x000F000Fu, mhi = 0x00F000F0u, mg = 0x64006400u;
     asm("" : "+v"(mlo), "+v"(mhi), "+v"(mg));
 
-    // the rows' scales 2^e (for the stores) read now, written to LDS after
-    // the loop: a buffer load, so no wait before the first stage covers them
-    float row_scale = 0.0f;
-    if (tid < BM && m0 + tid < ds.m)
-        row_scale = as_f32(bld4(make_rsrc(ds.xrs, 0xFFFFFFFFu), 4u * act_row(ds, m0 + tid)));
+    row_scale = row_scale_load(ds, m0, tid, BM);
     // prologue: stages 0-2 copied (with stage 0's Sx), stages 0-1's weights
     copy_act(0u, L.a[0], true);
     load_w(0u, true);
     copy_act(1u, L.a[1], false);
     copy_act(2u, L.a[2], false);
     Pipe::prologue_end();
-    u4_t q_odd[2] = {};  // the odd stage's operands, from the pair's swap
+    u4_t q_odd[NJ] = {};  // the odd stage's operands, from the pair's swap
     for (uint32_t st0 = 0; st0 < nst; st0 += 4u) {
 #pragma unroll
         for (uint32_t g = 0; g < 4u; g++) {
             const uint32_t st = st0 + g;
-            u4_t hdr[2];
+            u4_t hdr[NJ];
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
+            for (int j = 0; j < NJ; j++) {
                 if ((g & 1u) == 0u) {
 #pragma unroll
                     for (int d = 0; d < 4; d++) {
@@ -525,28 +527,27 @@ RFXQ_DEV void mmqh_q4k_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_
             if (g == 0u) {
                 // super-block start: the columns' multipliers, and the
                 // constant part C_b * Sx_b into the accumulators
-                u4_t cop[2];
+                u4_t cop[NJ];
 #pragma unroll
-                for (int j = 0; j < 2; j++) q4k_sb_operands(hdr[j], cop[j], dsc[j]);
+                for (int j = 0; j < NJ; j++) q4k_sb_operands(hdr[j], cop[j], dsc[j]);
 #pragma unroll
                 for (int i = 0; i < MT; i++) {
                     const u4_t sxo = L.sx[2u * (32u * i + l32) + h];
-                    acc[i][0] = mfma16(cop[0], sxo, acc[i][0]);
-                    acc[i][1] = mfma16(cop[1], sxo, acc[i][1]);
+                    for (int j = 0; j < NJ; j++) acc[i][j] = mfma16(cop[j], sxo, acc[i][j]);
                 }
             }
-            uint32_t sm[2][2];
+            uint32_t sm[2][NJ];
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
+            for (int j = 0; j < NJ; j++) {
                 sm[0][j] = splat16<0>(dsc[j][g]);
                 sm[1][j] = splat16<1>(dsc[j][g]);
             }
             // four 16-k steps t = 2e + s2 (block 2g + e, positions 16s2..),
             // software pipelined: the operands of step t + 1 are read and built
             // while the eight MFMAs of step t run
-            uint32_t qs8[2][4];
+            uint32_t qs8[NJ][4];
 #pragma unroll
-            for (int j = 0; j < 2; j++)
+            for (int j = 0; j < NJ; j++)
 #pragma unroll
                 for (int u = 0; u < 4; u++) qs8[j][u] = q[j][u] >> 8;
             auto wop = [&](int t, int j) {
@@ -555,25 +556,24 @@ RFXQ_DEV void mmqh_q4k_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_
                 return e ? q4k_codes_f16<1>(a0, a1, b0, b1, sm[1][j], mhi, mg)
                          : q4k_codes_f16<0>(a0, a1, b0, b1, sm[0][j], mlo, mg);
             };
-            u4_t Xc[MT], Wc[2];
+            u4_t Xc[MT], Wc[NJ];
 #pragma unroll
             for (int i = 0; i < MT; i++) Xc[i] = S16[256u * i + a_act[0][0]];
-            Wc[0] = wop(0, 0);
-            Wc[1] = wop(0, 1);
+#pragma unroll
+            for (int j = 0; j < NJ; j++) Wc[j] = wop(0, j);
 #pragma unroll
             for (int t = 0; t < 4; t++) {
-                u4_t Xn[MT], Wn[2];
+                u4_t Xn[MT], Wn[NJ];
                 if (t < 3) {
                     const int e = (t + 1) >> 1, s2 = (t + 1) & 1;
 #pragma unroll
                     for (int i = 0; i < MT; i++) Xn[i] = S16[256u * i + a_act[e][s2]];
-                    Wn[0] = wop(t + 1, 0);
-                    Wn[1] = wop(t + 1, 1);
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) Wn[j] = wop(t + 1, j);
                 }
 #pragma unroll
                 for (int i = 0; i < MT; i++) {
-                    acc[i][0] = mfma16(Wc[0], Xc[i], acc[i][0]);
-                    acc[i][1] = mfma16(Wc[1], Xc[i], acc[i][1]);
+                    for (int j = 0; j < NJ; j++) acc[i][j] = mfma16(Wc[j], Xc[i], acc[i][j]);
                 }
                 if (t < 3) {
                     // interleave: per MFMA one LDS read (first MT) and a few VALU ops
@@ -591,8 +591,8 @@ RFXQ_DEV void mmqh_q4k_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                     for (int i = 0; i < MT; i++) Xc[i] = Xn[i];
-                    Wc[0] = Wn[0];
-                    Wc[1] = Wn[1];
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) Wc[j] = Wn[j];
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -604,68 +604,97 @@ RFXQ_DEV void mmqh_q4k_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_
     }
     // no copy may land in LDS after the workgroup is gone
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (tid < BM) L.sc[tid] = row_scale;
-    lds_barrier();
+}
 
-    float* y = ds.y + (uint64_t)ks * ds.m * ds.ldy;
-    if (!pair) {
-        store_wave<MT>(ds, y, m0, n0 + 64u * w, acc, L.sc, pick_buf(L.a[0], L.a[1], L.a[2], L.a[3], w));
-        return;
-    }
-    // gate/up pair: the two waves of a 64-column block split the epilogue.
-    // The gate wave passes its j = 1 tiles to the up wave, the up wave its
-    // j = 0 tiles to the gate wave, through the stage buffers (tile (i, j) of
-    // the block c in buffer 2c + j at 4 KB i, each lane's 16 values at 64
-    // bytes lane: both waves' accumulators have one layout); each then
-    // stores s = silu(g) * u for its 32 columns, g and u the scaled outputs
-    // (silu_and_mul.cu:7-23: g / (1 + expf(-g)) * u), unscaled.
-    const int keep = upw ? 1 : 0;  // the j-tile this wave finishes
+namespace mmqh {
+// A 32x32 tile's accumulator passed between waves through 4 KB of LDS, four
+// values a lane at a time, consecutive lanes 16 bytes apart
+RFXQ_DEV void pass_tile(float* b, const v16f_t& v) {
+    const uint32_t lane = threadIdx.x & 63u;
 #pragma unroll
-    for (int i = 0; i < MT; i++) {
-        float* b = reinterpret_cast<float*>(pick_buf(L.a[0], L.a[1], L.a[2], L.a[3], 2u * wc + (1u - keep))) +
-                   1024u * i + 16u * lane;
-        const v16f_t& v = acc[i][1 - keep];
+    for (int r = 0; r < 4; r++)
+        *reinterpret_cast<f4v_t*>(b + 256 * r + 4u * lane) = f4v_t{v[4 * r], v[4 * r + 1], v[4 * r + 2], v[4 * r + 3]};
+}
+RFXQ_DEV f4v_t passed(const float* b, int r) {
+    return *reinterpret_cast<const f4v_t*>(b + 256 * r + 4u * (threadIdx.x & 63u));
+}
+}  // namespace mmqh
+
+// A gate/up pair's epilogue: waves 0-1 hold gate columns, waves 2-3 the same
+// columns of up, and the two waves of a 64-column block split it. The gate
+// wave (KEEP = 0) passes its j = 1 tiles to the up wave (KEEP = 1), the up
+// wave its j = 0 tiles to the gate wave, through the stage buffers (tile
+// (i, j) of block c in buffer 2c + j at 4 KB i); each then stores
+// s = silu(g) * u for its 32 columns, g and u the scaled outputs
+// (silu_and_mul.cu:7-23: g / (1 + expf(-g)) * u), unscaled.
+template <int MT, int KEEP>
+RFXQ_DEV void mmqh_pair_store(const MmqDesc& ds, uint32_t m0, uint32_t n0, const mmqh::ActLds& L,
+                              v16f_t (&acc)[MT][2]) {
+    using namespace mmqh;
+    const uint32_t h = (threadIdx.x >> 5) & 1u, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wc = w & 1u;  // the wave's 64-column block
+    auto tile = [&](int i, int j) {
+        return reinterpret_cast<float*>(pick_buf(L.a[0], L.a[1], L.a[2], L.a[3], 2u * wc + j)) + 1024u * i;
+    };
 #pragma unroll
-        for (int r = 0; r < 16; r += 4) *reinterpret_cast<f4v_t*>(b + r) = f4v_t{v[r], v[r + 1], v[r + 2], v[r + 3]};
-    }
+    for (int i = 0; i < MT; i++) pass_tile(tile(i, 1 - KEEP), acc[i][1 - KEEP]);
     lds_barrier();
     {
 #pragma clang fp contract(off)
 #pragma unroll
-        for (int i = 0; i < MT; i++) {
-            const float* b = reinterpret_cast<const float*>(pick_buf(L.a[0], L.a[1], L.a[2], L.a[3], 2u * wc + keep)) +
-                             1024u * i + 16u * lane;
+        for (int i = 0; i < MT; i++)
 #pragma unroll
             for (int q4 = 0; q4 < 4; q4++) {
-                const f4v_t pv = *reinterpret_cast<const f4v_t*>(b + 4 * q4);
+                const f4v_t pv = passed(tile(i, KEEP), q4);
                 const float4 s4 = *reinterpret_cast<const float4*>(L.sc + 32u * i + 4u * h + 8u * q4);
                 const float sv[4] = {s4.x, s4.y, s4.z, s4.w};
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
-                    const float mine = acc[i][keep][4 * q4 + r] * sv[r], other = pv[r] * sv[r];
-                    const float g = upw ? other : mine, u = upw ? mine : other;
-                    acc[i][keep][4 * q4 + r] = (g / (1.0f + expf(-g))) * u;
+                    const float mine = acc[i][KEEP][4 * q4 + r] * sv[r], other = pv[r] * sv[r];
+                    const float g = KEEP ? other : mine, u = KEEP ? mine : other;
+                    acc[i][KEEP][4 * q4 + r] = (g / (1.0f + expf(-g))) * u;
                 }
             }
-        }
     }
     lds_barrier();  // every passed tile read before the stores reuse the buffers
-    if (upw)
-        store_wave<MT, 2>(ds, y, m0, n0 + 64u * wc, acc, L.sc, pick_buf(L.a[0], L.a[1], L.a[2], L.a[3], w), false);
-    else
-        store_wave<MT, 1>(ds, y, m0, n0 + 64u * wc, acc, L.sc, pick_buf(L.a[0], L.a[1], L.a[2], L.a[3], w), false);
+    store_wave<MT, 2, 1 << KEEP>(ds, ds.y, m0, n0 + 64u * wc, acc, L.sc, pick_buf(L.a[0], L.a[1], L.a[2], L.a[3], w), false);
 }
 
-template <int MT>
-RFXQ_DEV void mmqh_q6k_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_t ks, const mmqh::ActLds& ls);
-template <int MT>
-RFXQ_DEV void mmqh_q80_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_t ks, const mmqh::ActLds& lds);
+template <int MT, int NJ>
+RFXQ_DEV void mmqh_q6k_acc(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_t sb0, uint32_t sb1,
+                           const mmqh::ActLds& ls, v16f_t (&acc)[MT][NJ], float& row_scale);
+template <int MT, int NJ>
+RFXQ_DEV void mmqh_q80_acc(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_t sb0, uint32_t sb1,
+                           const mmqh::ActLds& ls, v16f_t (&acc)[MT][NJ], float& row_scale);
 
-// One (32 MT)x256 tile (and one split-K range): the descriptor made uniform,
+// The rows of one tile and split-K range: the accumulators, then the stores.
+template <int MT, int NJ, int TY>
+RFXQ_DEV void mmqh_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_t ks, const mmqh::ActLds& L) {
+    using namespace mmqh;
+    const uint32_t tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t sb0 = ks * ds.sb_per_split, sb1 = min(ds.k / 256u, sb0 + ds.sb_per_split);
+    v16f_t acc[MT][NJ];
+    float row_scale;
+    if constexpr (TY == TY_Q4K) mmqh_q4k_acc<MT, NJ>(ds, m0, n0, sb0, sb1, L, acc, row_scale);
+    else if constexpr (TY == TY_Q6K) mmqh_q6k_acc<MT, NJ>(ds, m0, n0, sb0, sb1, L, acc, row_scale);
+    else mmqh_q80_acc<MT, NJ>(ds, m0, n0, sb0, sb1, L, acc, row_scale);
+    if (tid < Tile<MT>::BM) L.sc[tid] = row_scale;
+    lds_barrier();
+    if constexpr (TY == TY_Q4K && NJ == 2)
+        if (ds.gu_pair != 0u) {
+            if (w >= 2u) mmqh_pair_store<MT, 1>(ds, m0, n0, L, acc);
+            else mmqh_pair_store<MT, 0>(ds, m0, n0, L, acc);
+            return;
+        }
+    store_wave<MT, NJ>(ds, ds.y + (uint64_t)ks * ds.m * ds.ldy, m0, n0 + 32u * NJ * w, acc, L.sc,
+                       pick_buf(L.a[0], L.a[1], L.a[2], L.a[3], w));
+}
+
+// One (32 MT) x (128 NJ) tile (and one split-K range): the descriptor made uniform,
 // the tile decoded, and the rows computed by the body of as many 32-row tiles
 // as the tile has rows (a ragged last tile, or an expert group of 33 rows in
 // a 64-row tile, runs no MFMAs on absent rows).
-template <int MT, int TY>
+template <int MT, int TY, int NJ = 2>
 RFXQ_DEV void mmqh_tile(const MmqDesc& dv, uint32_t t_local, const mmqh::ActLds& lds) {
     MmqDesc ds = dv;
     {
@@ -677,13 +706,11 @@ RFXQ_DEV void mmqh_tile(const MmqDesc& dv, uint32_t t_local, const mmqh::ActLds&
     const uint32_t ks = t_local % ds.splits;
     const uint32_t rest = t_local / ds.splits;
     const uint32_t tm = rest % ds.tiles_m, tn = rest / ds.tiles_m;
-    const uint32_t m0 = tm * 32u * MT, n0 = tn * (ds.gu_pair ? mmqh::BN / 2u : mmqh::BN);
+    const uint32_t m0 = tm * 32u * MT, n0 = tn * (NJ == 1 || ds.gu_pair ? 128u : 256u);
     const uint32_t sub = min((uint32_t)MT, (ds.m - m0 + 31u) / 32u);  // 32-row tiles with rows
     auto run = [&](auto mt) {
         constexpr int M = decltype(mt)::value;
-        if constexpr (TY == TY_Q4K) mmqh_q4k_rows<M>(ds, m0, n0, ks, lds);
-        else if constexpr (TY == TY_Q6K) mmqh_q6k_rows<M>(ds, m0, n0, ks, lds);
-        else mmqh_q80_rows<M>(ds, m0, n0, ks, lds);
+        mmqh_rows<M, NJ, TY>(ds, m0, n0, ks, lds);
     };
     if constexpr (MT >= 4) {
         if (sub >= 4u) return run(std::integral_constant<int, 4>{});
@@ -718,21 +745,19 @@ RFXQ_MMQH_ENTRY(rfxq_mmqh_q4k, TY_Q4K, 4, 2)
 RFXQ_MMQH_ENTRY(rfxq_mmqh_q4k_m32, TY_Q4K, 1, 4)
 RFXQ_MMQH_ENTRY(rfxq_mmqh_q4k_m64, TY_Q4K, 2, 3)
 
-// One (32 MT)x256 tile (and one split-K range) of Y = X . W^T for Q6_K weights:
+// Accumulators of one (32 MT) x (128 NJ) tile over super-blocks [sb0, sb1) for Q6_K weights:
 // the Q4_K tile's layout and pipeline, with the Q6_K weight operands.
-template <int MT>
-RFXQ_DEV void mmqh_q6k_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_t ks, const mmqh::ActLds& ls) {
+template <int MT, int NJ>
+RFXQ_DEV void mmqh_q6k_acc(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_t sb0, uint32_t sb1,
+                           const mmqh::ActLds& ls, v16f_t (&acc)[MT][NJ], float& row_scale) {
     using namespace mmqh;
-    constexpr uint32_t BM = Tile<MT>::BM;
     // weight loads per stage: the ql pieces; the qh pieces at even positions;
     // the scales and d at position 0
     constexpr int WA = MT == 4 ? 1 : 2;  // (128-row tiles: two stages of registers would spill)
-    using Pipe = StagePipe<MT, WA, 8, 2, 4, 2, 0>;
+    using Pipe = StagePipe<MT, WA, 4 * NJ, NJ, 2 * NJ, NJ, 0>;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, l32 = lane & 31u, h = lane >> 5;
     const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t nsb = ds.k / 256u;
-    const uint32_t sb0 = ks * ds.sb_per_split;
-    const uint32_t sb1 = min(nsb, sb0 + ds.sb_per_split);
     const uint32_t row_bytes = nsb * 210u;  // 2 mod 4 for an odd nsb
 
     // The weights' buffer starts at the dword at or below the tile's first
@@ -743,7 +768,7 @@ RFXQ_DEV void mmqh_q6k_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_
     const uint32_t sh0 = (uint32_t)(wa & 3u);
     const uint32_t rb = act_base(ds, m0);
     const rsrc_t r_act = make_rsrc(ds.xq + (uint64_t)rb * ds.ldq, 0xFFFFFFFFu);
-    const rsrc_t r_w = make_rsrc(reinterpret_cast<const void*>(wa - sh0), min(BN, ds.n - n0) * row_bytes + sh0);
+    const rsrc_t r_w = make_rsrc(reinterpret_cast<const void*>(wa - sh0), min(128u * NJ, ds.n - n0) * row_bytes + sh0);
     const uint32_t ra = tid >> 3;
     // activations: the Q4_K tile's staging, but the stage's logical chunks 4-7
     // (group B) sit 128 bytes after chunks 0-3 (group A) in the f16 row
@@ -755,18 +780,18 @@ RFXQ_DEV void mmqh_q6k_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_
     // stage, positions [16h, 16h + 16) of the ql and qh pieces of column
     // 64w + 32j + l32 (five dwords each), and with the first stage of a
     // super-block its scales and d.
-    uint32_t col[2], g_c[2];
+    uint32_t col[NJ], g_c[NJ];
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        col[j] = 64u * w + 32u * j + l32;
+    for (int j = 0; j < NJ; j++) {
+        col[j] = 32u * NJ * w + 32u * j + l32;
         g_c[j] = col[j] * row_bytes + 16u * h;
     }
     const uint32_t nst = 4u * (sb1 - sb0);
 
     // ql pieces of WA stages (by stage); qh, scales and d are copied out in
     // the stage that issues their next load
-    u4_t qln[WA][2], qhn[2], scn[2];
-    uint32_t dn[2];
+    u4_t qln[WA][NJ], qhn[NJ], scn[NJ];
+    uint32_t dn[NJ];
     auto copy_act = [&](uint32_t st, u4_t* buf) {
         const uint32_t sl = min(st, nst - 1u);
         const uint32_t sb = sb0 + (sl >> 2), g = sl & 3u;
@@ -784,33 +809,31 @@ RFXQ_DEV void mmqh_q6k_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_
         const uint32_t base = 210u * sb + sh0;
         // the qh piece of half n serves both of its stages: loaded with s = 0
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
+        for (int j = 0; j < NJ; j++) {
             qln[st % WA][j] = __builtin_amdgcn_raw_buffer_load_b128(r_w, g_c[j], base + 64u * n + 32u * s, 0);
             if ((st & 1u) == 0u) qhn[j] = __builtin_amdgcn_raw_buffer_load_b128(r_w, g_c[j], base + 128u + 32u * n, 0);
         }
         if ((st & 3u) == 0u) {
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
+            for (int j = 0; j < NJ; j++) {
                 scn[j] = __builtin_amdgcn_raw_buffer_load_b128(r_w, g_c[j] - 16u * h, base + 192u, 0);
                 dn[j] = __builtin_amdgcn_raw_buffer_load_b16(r_w, g_c[j] - 16u * h, base + 208u, 0);
             }
         }
     };
 
-    v16f_t acc[MT][2];
 #pragma unroll
-    for (int i = 0; i < MT; i++) acc[i][0] = acc[i][1] = v16f_t{};
+    for (int i = 0; i < MT; i++) for (int j = 0; j < NJ; j++) acc[i][j] = v16f_t{};
     uint32_t a_act[2][2];
 #pragma unroll
     for (int e = 0; e < 2; e++)
 #pragma unroll
         for (int s2 = 0; s2 < 2; s2++) a_act[e][s2] = l32 * 8u + ((4u * e + 2u * h + s2) ^ ((l32 >> 1) & 7u));
-    u4_t mult[2] = {}, L[2], Q[2];
+    u4_t mult[NJ] = {}, L[NJ], Q[NJ];
     uint32_t mla = 0x000F000Fu, mqa = 0x00300030u, mlb = 0x00F000F0u, mqb = 0x03000300u, mg = 0x64006400u;
     asm("" : "+v"(mla), "+v"(mqa), "+v"(mlb), "+v"(mqb), "+v"(mg));
 
-    float row_scale = 0.0f;  // written to LDS after the loop (as for Q4_K)
-    if (tid < BM && m0 + tid < ds.m) row_scale = as_f32(bld4(make_rsrc(ds.xrs, 0xFFFFFFFFu), 4u * act_row(ds, m0 + tid)));
+    row_scale = row_scale_load(ds, m0, tid, Tile<MT>::BM);
     copy_act(0u, ls.a[0]);
     if constexpr (WA == 1) {
         copy_act(1u, ls.a[1]);
@@ -828,7 +851,7 @@ RFXQ_DEV void mmqh_q6k_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_
             const uint32_t st = st0 + g;
             const uint32_t n = g >> 1, s = g & 1u;
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
+            for (int j = 0; j < NJ; j++) {
                 L[j] = qln[g % WA][j];
                 if (s == 0u) Q[j] = qhn[j];
                 if (g == 0u) mult[j] = q6k_multipliers(scn[j], dn[j], h);
@@ -837,16 +860,16 @@ RFXQ_DEV void mmqh_q6k_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_
             copy_act(st + 3u, ls.a[(g + 3u) & 3u]);
             const u4_t* S16 = ls.a[g];
             // groups A (e = 0) and B (e = 1): multipliers i = 4n + s + 2e
-            uint32_t sm[2][2];
+            uint32_t sm[2][NJ];
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
+            for (int j = 0; j < NJ; j++) {
                 sm[0][j] = s ? splat16<1>(mult[j][2 * n]) : splat16<0>(mult[j][2 * n]);
                 sm[1][j] = s ? splat16<1>(mult[j][2 * n + 1]) : splat16<0>(mult[j][2 * n + 1]);
             }
             // shifted copies of the stage's code dwords (see q6k_codes_f16)
-            uint32_t Ls[2][4], Qa[2][4], Qb[2][4];
+            uint32_t Ls[NJ][4], Qa[NJ][4], Qb[NJ][4];
 #pragma unroll
-            for (int j = 0; j < 2; j++)
+            for (int j = 0; j < NJ; j++)
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
                     Ls[j][u] = L[j][u] >> 8;
@@ -861,25 +884,24 @@ RFXQ_DEV void mmqh_q6k_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_
                 return q6k_codes_f16<1>(L[j][u], L[j][u + 1], Ls[j][u], Ls[j][u + 1], Qa[j][u], Qa[j][u + 1],
                                         Qb[j][u], Qb[j][u + 1], sm[1][j], mlb, mqb, mg);
             };
-            u4_t Xc[MT], Wc[2];
+            u4_t Xc[MT], Wc[NJ];
 #pragma unroll
             for (int i = 0; i < MT; i++) Xc[i] = S16[256u * i + a_act[0][0]];
-            Wc[0] = wop(0, 0);
-            Wc[1] = wop(0, 1);
+#pragma unroll
+            for (int j = 0; j < NJ; j++) Wc[j] = wop(0, j);
 #pragma unroll
             for (int t = 0; t < 4; t++) {
-                u4_t Xn[MT], Wn[2];
+                u4_t Xn[MT], Wn[NJ];
                 if (t < 3) {
                     const int e = (t + 1) >> 1, s2 = (t + 1) & 1;
 #pragma unroll
                     for (int i = 0; i < MT; i++) Xn[i] = S16[256u * i + a_act[e][s2]];
-                    Wn[0] = wop(t + 1, 0);
-                    Wn[1] = wop(t + 1, 1);
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) Wn[j] = wop(t + 1, j);
                 }
 #pragma unroll
                 for (int i = 0; i < MT; i++) {
-                    acc[i][0] = mfma16(Wc[0], Xc[i], acc[i][0]);
-                    acc[i][1] = mfma16(Wc[1], Xc[i], acc[i][1]);
+                    for (int j = 0; j < NJ; j++) acc[i][j] = mfma16(Wc[j], Xc[i], acc[i][j]);
                 }
                 if (t < 3) {
 #pragma unroll
@@ -896,8 +918,8 @@ RFXQ_DEV void mmqh_q6k_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                     for (int i = 0; i < MT; i++) Xc[i] = Xn[i];
-                    Wc[0] = Wn[0];
-                    Wc[1] = Wn[1];
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) Wc[j] = Wn[j];
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -906,12 +928,6 @@ RFXQ_DEV void mmqh_q6k_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_
     }
     // no copy may land in LDS after the workgroup is gone
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (tid < BM) ls.sc[tid] = row_scale;
-    lds_barrier();
-
-    float* y = ds.y + (uint64_t)ks * ds.m * ds.ldy;
-    const float* sc = ls.sc;
-    store_wave<MT>(ds, y, m0, n0 + 64u * w, acc, sc, pick_buf(ls.a[0], ls.a[1], ls.a[2], ls.a[3], w));
 }
 
 RFXQ_MMQH_ENTRY(rfxq_mmqh_q6k, TY_Q6K, 4, 2)
@@ -948,21 +964,19 @@ RFXQ_DEV u2_t q80_codes_f16(uint32_t v, h2_t dv, uint32_t mg) {
 }
 }  // namespace mmqh
 
-// One (32 MT)x256 tile (and one split-K range) of Y = X . W^T for Q8_0 weights:
+// Accumulators of one (32 MT) x (128 NJ) tile over [sb0, sb1) (256 values each) for Q8_0 weights:
 // the Q4_K tile's activation staging and MFMA schedule, with Q8_0 operands.
-template <int MT, bool AL>
-RFXQ_DEV void mmqh_q80_rows_t(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_t ks, const mmqh::ActLds& ls) {
+template <int MT, int NJ, bool AL>
+RFXQ_DEV void mmqh_q80_acc_t(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_t sb0, uint32_t sb1,
+                             const mmqh::ActLds& ls, v16f_t (&acc)[MT][NJ], float& row_scale) {
     using namespace mmqh;
-    constexpr uint32_t BM = Tile<MT>::BM;
     // weights two stages ahead in the 96- and 128-row bodies; one in the
     // smaller ones, whose entries cap the registers lower
     constexpr int WA = MT >= 3 ? 2 : 1;
-    using Pipe = StagePipe<MT, WA, 8, 8, 8, 8, 0>;  // weight loads: four per column and stage
+    using Pipe = StagePipe<MT, WA, 4 * NJ, 4 * NJ, 4 * NJ, 4 * NJ, 0>;  // weight loads: four per column and stage
     const uint32_t tid = threadIdx.x, lane = tid & 63u, l32 = lane & 31u, h = lane >> 5;
     const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t nsb = ds.k / 256u;
-    const uint32_t sb0 = ks * ds.sb_per_split;
-    const uint32_t sb1 = min(nsb, sb0 + ds.sb_per_split);
     const uint32_t row_bytes = nsb * 272u;
 
     // weights: the dword at or below the tile's first column (2-byte aligned)
@@ -970,7 +984,7 @@ RFXQ_DEV void mmqh_q80_rows_t(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint3
     const uint32_t sh0 = (uint32_t)(wa & 3u);
     const uint32_t rb = act_base(ds, m0);
     const rsrc_t r_act = make_rsrc(ds.xq + (uint64_t)rb * ds.ldq, 0xFFFFFFFFu);
-    const rsrc_t r_w = make_rsrc(reinterpret_cast<const void*>(wa - sh0), min(BN, ds.n - n0) * row_bytes + sh0);
+    const rsrc_t r_w = make_rsrc(reinterpret_cast<const void*>(wa - sh0), min(128u * NJ, ds.n - n0) * row_bytes + sh0);
     const uint32_t ra = tid >> 3;
     uint32_t g_act[MT];
 #pragma unroll
@@ -979,10 +993,10 @@ RFXQ_DEV void mmqh_q80_rows_t(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint3
     // each block, and each block's d
     // (the lane-varying parts of an offset go in the VGPR offset: a
     // lane-varying SGPR offset would make the compiler loop over lanes)
-    uint32_t g_c[2], g_q[2];
+    uint32_t g_c[NJ], g_q[NJ];
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        g_c[j] = (64u * w + 32u * j + l32) * row_bytes + sh0;
+    for (int j = 0; j < NJ; j++) {
+        g_c[j] = (32u * NJ * w + 32u * j + l32) * row_bytes + sh0;
         g_q[j] = g_c[j] + (AL ? 16u * h : 2u + 16u * h);
     }
     const uint32_t e_off = h ? 0u : 32u;  // aligned form: the dword with the other half's d
@@ -992,8 +1006,8 @@ RFXQ_DEV void mmqh_q80_rows_t(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint3
     // form qn = codes of blocks 0, 1 and dn = their d; aligned form qn[0] =
     // bytes [16h, +16), qn[1] = bytes [36 + 16h, +16), dn[0] = the dword after
     // qn[0], dn[1] = the other d's dword
-    u4_t qn_[WA][2][2];
-    uint32_t dn_[WA][2][2];
+    u4_t qn_[WA][NJ][2];
+    uint32_t dn_[WA][NJ][2];
     auto copy_act = [&](uint32_t st, u4_t* buf) {
         const uint32_t sl = min(st, nst - 1u);
         const uint32_t sb = sb0 + (sl >> 2), g = sl & 3u;
@@ -1010,7 +1024,7 @@ RFXQ_DEV void mmqh_q80_rows_t(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint3
         if constexpr (AL) {
             const uint32_t o = 34u * blk;  // dword aligned (blk is even)
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
+            for (int j = 0; j < NJ; j++) {
                 qn[j][0] = __builtin_amdgcn_raw_buffer_load_b128(r_w, g_q[j], o, 0);
                 dn[j][0] = __builtin_amdgcn_raw_buffer_load_b32(r_w, g_q[j], o + 16u, 0);
                 qn[j][1] = __builtin_amdgcn_raw_buffer_load_b128(r_w, g_q[j], o + 36u, 0);
@@ -1018,7 +1032,7 @@ RFXQ_DEV void mmqh_q80_rows_t(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint3
             }
         } else {
 #pragma unroll
-            for (int j = 0; j < 2; j++)
+            for (int j = 0; j < NJ; j++)
 #pragma unroll
                 for (int e = 0; e < 2; e++) {
                     const uint32_t o = 34u * (blk + e);
@@ -1028,9 +1042,8 @@ RFXQ_DEV void mmqh_q80_rows_t(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint3
         }
     };
 
-    v16f_t acc[MT][2];
 #pragma unroll
-    for (int i = 0; i < MT; i++) acc[i][0] = acc[i][1] = v16f_t{};
+    for (int i = 0; i < MT; i++) for (int j = 0; j < NJ; j++) acc[i][j] = v16f_t{};
     uint32_t a_act[2][2];
 #pragma unroll
     for (int e = 0; e < 2; e++)
@@ -1039,8 +1052,7 @@ RFXQ_DEV void mmqh_q80_rows_t(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint3
     uint32_t mg = 0x64646464u, sgn = 0x80808080u;
     asm("" : "+v"(mg), "+v"(sgn));
 
-    float row_scale = 0.0f;  // written to LDS after the loop (as for Q4_K)
-    if (tid < BM && m0 + tid < ds.m) row_scale = as_f32(bld4(make_rsrc(ds.xrs, 0xFFFFFFFFu), 4u * act_row(ds, m0 + tid)));
+    row_scale = row_scale_load(ds, m0, tid, Tile<MT>::BM);
     copy_act(0u, ls.a[0]);
     if constexpr (WA == 1) {
         copy_act(1u, ls.a[1]);
@@ -1058,10 +1070,10 @@ RFXQ_DEV void mmqh_q80_rows_t(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint3
             const uint32_t st = st0 + g;
             const auto& qn = qn_[g % WA];
             const auto& dn = dn_[g % WA];
-            u4_t q[2][2];
-            h2_t dv[2][2];
+            u4_t q[NJ][2];
+            h2_t dv[NJ][2];
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
+            for (int j = 0; j < NJ; j++) {
                 if constexpr (AL) {
                     const u4_t a = qn[j][0];
                     const uint32_t b = dn[j][0], e = dn[j][1];
@@ -1087,25 +1099,24 @@ RFXQ_DEV void mmqh_q80_rows_t(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint3
                 const u2_t hi = q80_codes_f16(q[j][e][2 * s2 + 1], dv[j][e], mg);
                 return u4_t{lo.x, lo.y, hi.x, hi.y};
             };
-            u4_t Xc[MT], Wc[2];
+            u4_t Xc[MT], Wc[NJ];
 #pragma unroll
             for (int i = 0; i < MT; i++) Xc[i] = S16[256u * i + a_act[0][0]];
-            Wc[0] = wop(0, 0);
-            Wc[1] = wop(0, 1);
+#pragma unroll
+            for (int j = 0; j < NJ; j++) Wc[j] = wop(0, j);
 #pragma unroll
             for (int t = 0; t < 4; t++) {
-                u4_t Xn[MT], Wn[2];
+                u4_t Xn[MT], Wn[NJ];
                 if (t < 3) {
                     const int e = (t + 1) >> 1, s2 = (t + 1) & 1;
 #pragma unroll
                     for (int i = 0; i < MT; i++) Xn[i] = S16[256u * i + a_act[e][s2]];
-                    Wn[0] = wop(t + 1, 0);
-                    Wn[1] = wop(t + 1, 1);
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) Wn[j] = wop(t + 1, j);
                 }
 #pragma unroll
                 for (int i = 0; i < MT; i++) {
-                    acc[i][0] = mfma16(Wc[0], Xc[i], acc[i][0]);
-                    acc[i][1] = mfma16(Wc[1], Xc[i], acc[i][1]);
+                    for (int j = 0; j < NJ; j++) acc[i][j] = mfma16(Wc[j], Xc[i], acc[i][j]);
                 }
                 if (t < 3) {
 #pragma unroll
@@ -1122,8 +1133,8 @@ RFXQ_DEV void mmqh_q80_rows_t(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint3
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                     for (int i = 0; i < MT; i++) Xc[i] = Xn[i];
-                    Wc[0] = Wn[0];
-                    Wc[1] = Wn[1];
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) Wc[j] = Wn[j];
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -1132,18 +1143,13 @@ RFXQ_DEV void mmqh_q80_rows_t(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint3
     }
     // no copy may land in LDS after the workgroup is gone
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (tid < BM) ls.sc[tid] = row_scale;
-    lds_barrier();
-
-    float* y = ds.y + (uint64_t)ks * ds.m * ds.ldy;
-    const float* sc = ls.sc;
-    store_wave<MT>(ds, y, m0, n0 + 64u * w, acc, sc, pick_buf(ls.a[0], ls.a[1], ls.a[2], ls.a[3], w));
 }
 
-template <int MT>
-RFXQ_DEV void mmqh_q80_rows(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_t ks, const mmqh::ActLds& lds) {
-    if ((reinterpret_cast<uintptr_t>(ds.w) & 3u) == 0u) mmqh_q80_rows_t<MT, true>(ds, m0, n0, ks, lds);
-    else mmqh_q80_rows_t<MT, false>(ds, m0, n0, ks, lds);
+template <int MT, int NJ>
+RFXQ_DEV void mmqh_q80_acc(const MmqDesc& ds, uint32_t m0, uint32_t n0, uint32_t sb0, uint32_t sb1,
+                           const mmqh::ActLds& ls, v16f_t (&acc)[MT][NJ], float& row_scale) {
+    if ((reinterpret_cast<uintptr_t>(ds.w) & 3u) == 0u) mmqh_q80_acc_t<MT, NJ, true>(ds, m0, n0, sb0, sb1, ls, acc, row_scale);
+    else mmqh_q80_acc_t<MT, NJ, false>(ds, m0, n0, sb0, sb1, ls, acc, row_scale);
 }
 
 RFXQ_MMQH_ENTRY(rfxq_mmqh_q8_0, TY_Q8_0, 4, 2)
@@ -1178,3 +1184,34 @@ RFXQ_MMQH_ENTRY(rfxq_mmqh_q8_0_m64, TY_Q8_0, 2, 3)
         else mmqh_tile<MT, TY_Q4K>(d, b - d.wg_begin, lds);                                                    \
     }
 RFXQ_MMQH_MIX_ENTRY(rfxq_mmqh_mix_m32, 1, 3)
+
+// 64 x 128 tiles (32 columns a wave), any type: for GEMMs whose larger tiles
+// would be so few that K is cut into many ranges, whose partial sums then go
+// through memory (the host's choice, n128_better). A tile runs at two thirds
+// of the 128 x 256 tile's rate per CU (its weight operands serve 64 rows, its
+// activation reads 32 columns a wave), but there are four times as many: 512
+// rows of an 8B o_proj (4096 x 4096) take 28.6 us as 256 tiles, without a
+// reduce, against 30.6 us and a 15.5 us reduce as 512 ranges of 128 x 256
+// tiles. (64 x 256 tiles split four ways: 28.9 us and the reduce; two wave
+// groups per workgroup, each half of K, on any of these tiles: no faster.)
+#define RFXQ_MMQH_N128_ENTRY(NAME)                                                                          \
+    extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void NAME(MmqArgs args) { \
+        __shared__ __attribute__((aligned(16))) u4_t a0[mmqh::Tile<2>::kAct / 16u];                          \
+        __shared__ __attribute__((aligned(16))) u4_t a1[mmqh::Tile<2>::kAct / 16u];                          \
+        __shared__ __attribute__((aligned(16))) u4_t a2[mmqh::Tile<2>::kAct / 16u];                          \
+        __shared__ __attribute__((aligned(16))) u4_t a3[mmqh::Tile<2>::kAct / 16u];                          \
+        __shared__ __attribute__((aligned(16))) u4_t sx[mmqh::kThreads];                                     \
+        __shared__ __attribute__((aligned(16))) float sc[mmqh::Tile<2>::BM];                                 \
+        if (blockDim.x != mmqh::kThreads) return; /* the tile assumes exactly kThreads lanes */               \
+        const uint32_t tiles = min(gridDim.x, mmq_tile_count(args));                                        \
+        if (blockIdx.x >= tiles) return;                                                                     \
+        const uint32_t b = mmqh::xcd_tile(blockIdx.x, tiles);                                               \
+        const MmqDesc d = mmq_pick(args, b);                                                                 \
+        if (b - d.wg_begin >= d.tiles_m * d.tiles_n * d.splits) return;                                     \
+        const mmqh::ActLds lds{{a0, a1, a2, a3}, sx, sc};                                                    \
+        const uint32_t ty = __builtin_amdgcn_readfirstlane(d.type);                                         \
+        if (ty == TY_Q4K) mmqh_tile<2, TY_Q4K, 1>(d, b - d.wg_begin, lds);                                    \
+        else if (ty == TY_Q6K) mmqh_tile<2, TY_Q6K, 1>(d, b - d.wg_begin, lds);                               \
+        else mmqh_tile<2, TY_Q8_0, 1>(d, b - d.wg_begin, lds);                                                 \
+    }
+RFXQ_MMQH_N128_ENTRY(rfxq_mmqh_n128)

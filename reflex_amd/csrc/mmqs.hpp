@@ -370,7 +370,7 @@ RFXQ_DEV void tile(const MmqDesc& ds, uint32_t n0, uint32_t ks, uint8_t* lds) {
     }
     lds_barrier();  // every wave past its activations: their LDS takes the results
     float* y = ds.y + (uint64_t)ks * ds.m * ds.ldy;
-    store_wave<1>(ds, y, 0u, n0 + 64u * w, acc, L.sc, reinterpret_cast<u4_t*>(lds + 128u + 4096u * w));
+    store_wave<1, 2>(ds, y, 0u, n0 + 64u * w, acc, L.sc, reinterpret_cast<u4_t*>(lds + 128u + 4096u * w));
 }
 }  // namespace mmqs
 

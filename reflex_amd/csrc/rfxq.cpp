@@ -153,6 +153,7 @@ struct Ctx {
     hipFunction_t mmqh[3][3] = {};  // [Q4_K, Q6_K, Q8_0][128-row, 32-row, 64-row tiles]
     hipFunction_t mmqh_mix_m32 = nullptr;  // 32-row tiles, Q4_K or Q6_K per descriptor
     hipFunction_t mmqs = nullptr;          // up to 32 rows, any type per descriptor
+    hipFunction_t mmqh_n128 = nullptr;     // 64 x 128 tiles, any type per descriptor
     hipFunction_t act_f16 = nullptr, act_f16_multi = nullptr, act_f16_wg = nullptr, act_f16_multi_wg = nullptr;
     hipFunction_t deq[3][2] = {};
     hipFunction_t gather = nullptr, scatter = nullptr, silu = nullptr, combine = nullptr;
@@ -231,6 +232,7 @@ int load_ctx(int device, Ctx** out) {
         {&c->mmqh[2][2], "rfxq_mmqh_q8_0_m64"},
         {&c->mmqh_mix_m32, "rfxq_mmqh_mix_m32"},
         {&c->mmqs, "rfxq_mmqs"},
+        {&c->mmqh_n128, "rfxq_mmqh_n128"},
         {&c->act_f16, "rfxq_act_f16"},
         {&c->act_f16_multi, "rfxq_act_f16_multi"},
         {&c->act_f16_wg, "rfxq_act_f16_wg"},
@@ -949,6 +951,62 @@ uint32_t small_gemm_tile_m(uint32_t tile_m, uint32_t rows, uint32_t n, uint32_t 
     return tile_m;
 }
 
+// ---- 64 x 128 tiles instead of the larger ones
+//
+// Estimated time (us) of one f16 launch of GEMMs {n, super-blocks per row} of
+// `rows` rows on `bm` x `bn` tiles with ranges of `sb` super-blocks. A CU
+// takes `c` us per tile and super-block, whether its workgroups run side by
+// side or in turn; a launch of more workgroups than CUs ends later than its
+// average CU (fitted: 0.85 of the average load and 0.35 of a workgroup).
+// Partial sums of split GEMMs are written and read once at 5 TB/s.
+struct GemmShape {
+    uint32_t n, nsb;
+};
+double mmqh_time(const std::vector<GemmShape>& g, uint32_t rows, uint32_t bm, uint32_t bn, uint32_t sb, double c,
+                 uint32_t cus) {
+    uint64_t wgs = 0;
+    double load = 0.0, part = 0.0;
+    uint32_t longest = 0;
+    for (const auto& s : g) {
+        const uint64_t tiles = (uint64_t)((rows + bm - 1u) / bm) * ((s.n + bn - 1u) / bn);
+        const uint32_t splits = (s.nsb + sb - 1u) / sb;
+        wgs += tiles * splits;
+        load += (double)tiles * s.nsb;
+        longest = std::max(longest, std::min(sb, s.nsb));
+        if (splits > 1u) part += 8.0 * splits * rows * s.n / 5e6;
+    }
+    return 3.0 + part + c * (wgs <= cus ? longest : 0.85 * load / cus + 0.35 * longest);
+}
+
+// Super-blocks per range on 64 x 128 tiles for the GEMMs of one type and one
+// launch, or 0 where the larger tiles `base` {rows, super-blocks per range}
+// are estimated faster. 64 x 128 tiles split K only as far as there are idle
+// CUs. us per tile and super-block, measured (Q4_K / Q6_K / Q8_0): 128 x 256
+// 4.1 / 5.5 / 7.5, 64 x 256 2.9 / 4.0 / 4.5, 64 x 128 1.65 / 2.35 / 2.5; main
+// launch and reduce at 4096 x 4096 Q4_K: 64 rows 11.5 + 3.5 -> 8.1 + 3.5 us,
+// 128 rows 15.2 + 4.5 -> 10.9 + 3.5, 512 rows 30.6 + 15.5 -> 28.6 + 0, 1024
+// rows 42.9 + 10 -> 50.2 + 0; 4096 x 14336 Q6_K at 512 rows stays on 128 x 256
+// tiles (92 + 15 against 123).
+struct TileSplit {
+    uint32_t tile_m, sb;
+};
+uint32_t n128_sb(const std::vector<GemmShape>& g, uint32_t ty, uint32_t rows, uint32_t cus, TileSplit base) {
+    static const double kBig[3] = {4.1, 5.5, 7.5}, kMid[3] = {2.9, 4.0, 4.5}, kSmall[3] = {1.65, 2.35, 2.5};
+    if (rows <= 32u) return 0u;
+    const int t = type_index(ty);
+    std::vector<std::pair<uint32_t, uint32_t>> tiles;
+    uint32_t max_nsb = 1;
+    for (const auto& s : g) {
+        tiles.push_back({((rows + 63u) / 64u) * ((s.n + 127u) / 128u), s.nsb});
+        max_nsb = std::max(max_nsb, s.nsb);
+    }
+    const uint32_t sb = split_sb(tiles, 1u, std::max(1u, cus));
+    // 32-row tiles (small_gemm_tile_m): half a 64-row tile's weight operands at the least
+    const double big = mmqh_time(g, rows, base.tile_m, 256u, base.sb,
+                                 base.tile_m >= 128u ? kBig[t] : base.tile_m == 64u ? kMid[t] : 0.75 * kMid[t], cus);
+    return mmqh_time(g, rows, 64u, 128u, sb, kSmall[t], cus) < big ? sb : 0u;
+}
+
 // raw bytes of a weight matrix
 uint64_t gemm_weight_bytes(uint32_t ty, uint32_t k, uint32_t n) {
     return ty == RFXQ_TYPE_Q8_0 ? (uint64_t)n * (k / 32u) * 34u : (uint64_t)n * (k / 256u) * (ty == RFXQ_TYPE_Q6_K ? 210u : 144u);
@@ -1159,7 +1217,7 @@ int launch_combine(Ctx* c, const float* pair_out, const int32_t* idx, const floa
 bool mix_f16(uint32_t ty, uint32_t tile_m) { return (ty == RFXQ_TYPE_Q4_K || ty == RFXQ_TYPE_Q6_K) && tile_m == 32u; }
 
 int launch_mmq(Ctx* c, uint32_t ty, const MmqDesc* descs, uint32_t count, const MmqDesc* table, uint32_t total_wgs,
-               bool dots, hipStream_t stream, bool f16 = false, uint32_t tile_m = kMmqBM) {
+               bool dots, hipStream_t stream, bool f16 = false, uint32_t tile_m = kMmqBM, bool n128 = false) {
     const bool m64 = !f16 && tile_m == 64u;
     MmqArgs a;
     std::memset(&a, 0, sizeof a);
@@ -1169,7 +1227,7 @@ int launch_mmq(Ctx* c, uint32_t ty, const MmqDesc* descs, uint32_t count, const 
     hipFunction_t f = dots ? c->dots[type_index(ty)] : m64 ? c->mmq64[type_index(ty)] : c->mmq[type_index(ty)];
     // f16: Q4_K and Q6_K 32-row tiles mixed in one launch, others per type
     if (f16 && !dots)
-        f = mix_f16(ty, tile_m) ? c->mmqh_mix_m32 : c->mmqh[type_index(ty)][tile_m == 32u ? 1 : tile_m == 64u ? 2 : 0];
+        f = n128 ? c->mmqh_n128 : mix_f16(ty, tile_m) ? c->mmqh_mix_m32 : c->mmqh[type_index(ty)][tile_m == 32u ? 1 : tile_m == 64u ? 2 : 0];
     return launch(f, total_wgs, 0, stream, &a, sizeof a, "rfxq_mmq launch", kMmqThreads);
 }
 
@@ -1211,7 +1269,8 @@ int check_mmq_weight(const rfxq_weight* w, const char* what) {
 struct GemmPlan {
     rfxq_gemm_policy pol;
     bool f16 = false;
-    bool few = false;  // on rfxq_mmqs (which reads f32 activations: no layout)
+    bool few = false;   // on rfxq_mmqs (which reads f32 activations: no layout)
+    bool n128 = false;  // on 64 x 128 tiles
     uint32_t tiles_m = 1, tiles_n = 1;
     ActLayout act;
     uint64_t off_part = 0, total = 0;
@@ -1225,6 +1284,16 @@ GemmPlan plan_gemm(const Ctx* c, const rfxq_weight* w, uint32_t rows, const rfxq
     p.pol = gemm_policy(w->ggml_type, k, n, rows, c ? (uint32_t)c->cus : 256u, o);
     p.f16 = p.pol.path == PATH_MMQ_F16;
     if (p.pol.path == PATH_GEMV_ROWS) return p;  // no MMQ launch: tiles, layouts and workspace stay 0
+    const uint32_t cus = c ? (uint32_t)c->cus : 256u;
+    if (uint32_t sb = p.f16 && !o.quant_mma_splits ? n128_sb({{n, k / 256u}}, w->ggml_type, rows, cus,
+                                                             {p.pol.tile_m, p.pol.sb_per_split})
+                                                   : 0u) {
+        p.n128 = true;
+        p.pol.tile_m = 64u;
+        p.pol.tile_n = 128u;
+        p.pol.sb_per_split = sb;
+        p.pol.splits = (k / 256u + sb - 1u) / sb;
+    }
     p.tiles_m = (rows + p.pol.tile_m - 1u) / p.pol.tile_m;
     p.tiles_n = (n + p.pol.tile_n - 1u) / p.pol.tile_n;
     p.few = p.f16 && !in_place && p.pol.sb_per_split <= few_max_sb(rows);
@@ -1268,7 +1337,7 @@ int gemm_run(Ctx* c, const GemmPlan& p, const float* x, const uint8_t* act, cons
     d.sb_per_split = p.pol.sb_per_split;
     const uint32_t wgs = p.tiles_m * p.tiles_n * p.pol.splits;
     if (int rc = p.few ? launch_few(c, &d, 1, nullptr, wgs, stream)
-                       : launch_mmq(c, w->ggml_type, &d, 1, nullptr, wgs, false, stream, p.f16, p.pol.tile_m))
+                       : launch_mmq(c, w->ggml_type, &d, 1, nullptr, wgs, false, stream, p.f16, p.pol.tile_m, p.n128))
         return rc;
     if (p.pol.splits > 1)
         if (int rc = launch_reduce(c, part, y, (uint64_t)rows * n, p.pol.splits, stream)) return rc;
@@ -1307,8 +1376,9 @@ int check_act(const void* act, uint32_t rows, uint32_t k, const char* what) {
 // takes the single-GEMM policy's path (gemm_policy); GEMMs on the GEMV path
 // run as one GEMV per row in one table-driven launch.
 // type_index + 3 * variant (0: int8, 1: int8 64-row, 2: f16, 3: f16 32-row,
-// 4: f16 64-row); last the few-row kernel, every type
-constexpr uint32_t kGroupFew = 15, kGroupKernels = 16;
+// 4: f16 64-row); then the few-row kernel, every type
+// (15), then 64 x 128 tiles by type (16-18)
+constexpr uint32_t kGroupFew = 15, kGroupN128 = 16, kGroupKernels = 19;
 struct GemmGroup {
     struct Act {
         const float* x;
@@ -1341,8 +1411,10 @@ struct GemmGroup {
 bool group_f16(uint32_t g) { return g >= 6u; }
 uint32_t group_tile_m(uint32_t g) {
     const uint32_t v = g / 3u;
+    if (g >= kGroupN128) return 64u;
     return v == 1u || v == 4u ? 64u : v == 3u || v == 5u ? 32u : kMmqBM;
 }
+uint32_t group_tile_n(uint32_t g) { return g >= kGroupN128 ? 128u : tile_bn(group_f16(g)); }
 uint32_t group_variant(bool f16, uint32_t tile_m) { return f16 ? (tile_m == 32u ? 3u : tile_m == 64u ? 4u : 2u) : (tile_m == 64u ? 1u : 0u); }
 // the group (launch) of a GEMM: type_index + 3 * variant, except that the f16
 // 32-row tiles of Q4_K and Q6_K share one launch (rfxq_mmqh_mix_m32)
@@ -1409,6 +1481,27 @@ int build_gemm_group(const rfxq_gemm_item* items, uint32_t count, uint32_t rows,
         if (f16) g->acts[ai].need_h |= !few;
         else g->acts[ai].need_i8 = true;
     }
+    // the GEMMs of a type that 64 x 128 tiles are estimated to run faster
+    // than the launch's larger tiles (split as below)
+    for (uint32_t t = 6u; t < kGroupFew && !o.quant_mma_splits; t++) {
+        std::vector<GemmShape> shapes;
+        std::vector<std::pair<uint32_t, uint32_t>> tn;
+        uint32_t ty = 0, tiles = 0, max_nsb = 0;
+        for (uint32_t i = 0; i < count; i++) {
+            if (item_act[i] == ~0u || item_kernel[i] != t) continue;
+            ty = items[i].w->ggml_type;
+            shapes.push_back({items[i].w->out_features, items[i].w->in_features / 256u});
+            const uint32_t bm = group_tile_m(t);
+            tn.push_back({((rows + bm - 1u) / bm) * ((shapes.back().n + 255u) / 256u), shapes.back().nsb});
+            tiles += tn.back().first;
+            max_nsb = std::max(max_nsb, shapes.back().nsb);
+        }
+        if (shapes.empty()) continue;
+        const uint32_t sb = 2u * tiles < cus ? split_sb(tn, 2u, 2u * std::max(cus, 1u)) : max_nsb;
+        if (n128_sb(shapes, ty, rows, cus, {group_tile_m(t), sb}))
+            for (uint32_t i = 0; i < count; i++)
+                if (item_act[i] != ~0u && item_kernel[i] == t) item_kernel[i] = kGroupN128 + (uint32_t)type_index(ty);
+    }
     for (auto& a : g->acts) {
         if (a.ext) {
             a.L = act_layout(rows, a.k);
@@ -1434,7 +1527,7 @@ int build_gemm_group(const rfxq_gemm_item* items, uint32_t count, uint32_t rows,
         d.k = k;
         d.type = it.w->ggml_type;
         d.ldy = d.n;
-        const uint32_t bm = group_tile_m(t), bn = tile_bn(group_f16(t));
+        const uint32_t bm = group_tile_m(t), bn = group_tile_n(t);
         d.tiles_m = (rows + bm - 1u) / bm;
         d.tiles_n = (d.n + bn - 1u) / bn;
         d.splits = 1;
@@ -1450,12 +1543,13 @@ int build_gemm_group(const rfxq_gemm_item* items, uint32_t count, uint32_t rows,
     bool split_small[kGroupKernels] = {};
     for (uint32_t t = 0; t < kGroupKernels; t++) {
         auto& v = g->descs[t];
-        if (v.empty() || (!forced && 2u * g->wgs[t] >= cus && t != kGroupFew)) continue;
+        if (v.empty() || (!forced && 2u * g->wgs[t] >= cus && t < kGroupFew)) continue;
         split_small[t] = true;
         // one split size for the launch, so its workgroups take alike
         std::vector<std::pair<uint32_t, uint32_t>> tn;
         for (const auto& d : v) tn.push_back({d.tiles_m * d.tiles_n, d.k / 256u});
-        uint32_t w_sb = split_sb(tn, group_tile_m(t) == 32u ? 1u : 2u, 2u * std::max(cus, 1u));
+        uint32_t w_sb = t >= kGroupN128 ? split_sb(tn, 1u, std::max(cus, 1u))
+                                        : split_sb(tn, group_tile_m(t) == 32u ? 1u : 2u, 2u * std::max(cus, 1u));
         if (t == kGroupFew) w_sb = std::min(w_sb, few_max_sb(rows));
         uint32_t wg = 0;
         for (uint32_t i = 0; i < v.size(); i++) {
@@ -1543,7 +1637,7 @@ int launch_group_kernel(Ctx* c, const GemmGroup& g, uint32_t t, const MmqDesc* t
     if (v.empty()) return RFXQ_OK;
     if (t == kGroupFew) return launch_few(c, v.data(), (uint32_t)v.size(), table, g.wgs[t], stream);
     return launch_mmq(c, v[0].type, v.data(), (uint32_t)v.size(), table, g.wgs[t], false, stream, group_f16(t),
-                      group_tile_m(t));
+                      group_tile_m(t), t >= kGroupN128);
 }
 
 // the split-K reduces of kernel t
@@ -2038,7 +2132,7 @@ int rfxq_gemm_batch(const rfxq_gemm_item* items, uint32_t count, uint32_t rows, 
             }
             if (int rc = t == kGroupFew ? launch_few(c, d, cnt, nullptr, wg, stream)
                                         : launch_mmq(c, d[0].type, d, cnt, nullptr, wg, false, stream, group_f16(t),
-                                                     group_tile_m(t)))
+                                                     group_tile_m(t), t >= kGroupN128))
                 return rc;
         }
         if (int rc = run_group_reduces(c, g, t, stream)) return rc;

@@ -329,6 +329,27 @@ def test_gemm_few_rows_kernel(rq, orc, ty, m, n, k):
         assert np.abs(got - y).max() <= 1e-5 * np.abs(y).max()
 
 
+@pytest.mark.parametrize("ty", [Q4K, Q6K, Q8_0])
+@pytest.mark.parametrize("m,n,k", [(33, 129, 1280), (65, 640, 256), (100, 384, 2304), (333, 1030, 4096)])
+def test_gemm_64x128_tiles(rq, orc, opts, ty, m, n, k):
+    """64 x 128 tiles (GEMMs of few larger tiles): one and two 32-row sub-tiles, ragged columns (1030: dword
+    stores), split and unsplit K; the plain tiles (a forced split) agree to the rounding of the partial sums, a
+    grouped call and an activation buffer bit for bit."""
+    w_np = synth.weights(ty, n, k, 930 + m)
+    x_np = synth.activations(m * k, 931 + m).reshape(m, k)
+    y, _ = _check_gemm(rq, orc, ty, m, n, k, w_np, x_np)
+    x, w = _dev(x_np.reshape(-1)), _weight(rq, ty, w_np, n, k)
+    assert np.array_equal(rq.gemm_q8_1(rq.quantize_act_q8_1(x, m, k), w, m).cpu().numpy().reshape(m, n), y)
+    out = torch.full((m * n,), float("nan"), device=DEV)
+    plan = rq.GemmPlan([(x, w, out)], m)
+    for _ in range(2):
+        plan.run()
+        assert np.array_equal(out.cpu().numpy().reshape(m, n), y)
+    opts(quant_mma_splits=1)
+    plain = rq.gemm(x, w, m).cpu().numpy().reshape(m, n)
+    assert orc.rel_err_row_l2(y, plain.astype(np.float64)) < 1e-6
+
+
 def test_gemm_rows_independent_and_deterministic(rq, orc, opts):
     """Row r of the output depends only on row r of x, and repeats give identical bits."""
     n, k = 1024, 2048
