@@ -29,6 +29,38 @@ struct QuantSrcPlain {  // x[src_rows[r] or r][c], row stride ldx
     }
 };
 
+// One lane's four values of a 32-block (lane `part` of the block's 8; every
+// lane of the group calls): the codes to *q, the scales (lane 0) to *ds.
+RFXQ_DEV void q8_1_chunk(float4 v, uint32_t part, bool valid, int8_t* q, uint32_t* ds) {
+    float amax = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+    // the block's maximum in all 8 lanes (DPP within the lane group)
+    amax = fmaxf(amax, RFXQ_DPP(amax, 0xB1));
+    amax = fmaxf(amax, RFXQ_DPP(amax, 0x4E));
+    amax = fmaxf(amax, RFXQ_DPP(amax, 0x141));
+    const float d = amax / 127.0f;
+    const float id = d != 0.0f ? 1.0f / d : 0.0f;
+    const int q0 = (int)roundf(v.x * id), q1 = (int)roundf(v.y * id);
+    const int q2 = (int)roundf(v.z * id), q3 = (int)roundf(v.w * id);
+    float sum = ((v.x + v.y) + v.z) + v.w;
+    // lane distance 4, 2, 1 for the group's first lane (the one that
+    // stores it): row_shl:4, then quad_perm swaps of 2 and 1
+    sum += RFXQ_DPP(sum, 0x104);
+    sum += RFXQ_DPP(sum, 0x4E);
+    sum += RFXQ_DPP(sum, 0xB1);
+    if (valid) {
+        *reinterpret_cast<uint32_t*>(q) = (uint32_t)(q0 & 0xFF) | ((uint32_t)(q1 & 0xFF) << 8) |
+                                          ((uint32_t)(q2 & 0xFF) << 16) | ((uint32_t)(q3 & 0xFF) << 24);
+        if (part == 0u) {
+            const uint32_t dbits = __builtin_bit_cast(uint16_t, (half_t)d);
+            // round the product to f32 first (no fused single-rounding mixed mad)
+            float sid = sum * id;
+            asm volatile("" : "+v"(sid));
+            const uint32_t sbits = __builtin_bit_cast(uint16_t, (half_t)sid);
+            *ds = dbits | (sbits << 16);
+        }
+    }
+}
+
 // Rows [0, rows) of one activation, spread over `nwaves` waves (this one is
 // wave_global); 8 lanes per 32-block. `yout` (optional) receives the values
 // quantized, f32 [rows][k] (the producer's own output).
@@ -47,34 +79,7 @@ RFXQ_DEV void quant_q8_1_rows(const Src& src, uint32_t rows, uint32_t k, int8_t*
         const uint32_t part = lane & 7u;
         const float4 v = src.load(row, 32u * blk + 4u * part);
         if (yout && valid) *reinterpret_cast<float4*>(yout + (uint64_t)row * k + 32u * blk + 4u * part) = v;
-        float amax = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
-        // the block's maximum in all 8 lanes (DPP within the lane group)
-        amax = fmaxf(amax, RFXQ_DPP(amax, 0xB1));
-        amax = fmaxf(amax, RFXQ_DPP(amax, 0x4E));
-        amax = fmaxf(amax, RFXQ_DPP(amax, 0x141));
-        const float d = amax / 127.0f;
-        const float id = d != 0.0f ? 1.0f / d : 0.0f;
-        const int q0 = (int)roundf(v.x * id), q1 = (int)roundf(v.y * id);
-        const int q2 = (int)roundf(v.z * id), q3 = (int)roundf(v.w * id);
-        float sum = ((v.x + v.y) + v.z) + v.w;
-        // lane distance 4, 2, 1 for the group's first lane (the one that
-        // stores it): row_shl:4, then quad_perm swaps of 2 and 1
-        sum += RFXQ_DPP(sum, 0x104);
-        sum += RFXQ_DPP(sum, 0x4E);
-        sum += RFXQ_DPP(sum, 0xB1);
-        if (valid) {
-            const uint32_t packed = (uint32_t)(q0 & 0xFF) | ((uint32_t)(q1 & 0xFF) << 8) |
-                                    ((uint32_t)(q2 & 0xFF) << 16) | ((uint32_t)(q3 & 0xFF) << 24);
-            *reinterpret_cast<uint32_t*>(xq + (uint64_t)row * ldq + 32u * blk + 4u * part) = packed;
-            if (part == 0u) {
-                const uint32_t dbits = __builtin_bit_cast(uint16_t, (half_t)d);
-                // round the product to f32 first (no fused single-rounding mixed mad)
-                float sid = sum * id;
-                asm volatile("" : "+v"(sid));
-                const uint32_t sbits = __builtin_bit_cast(uint16_t, (half_t)sid);
-                xds[(uint64_t)row * nblk + blk] = dbits | (sbits << 16);
-            }
-        }
+        q8_1_chunk(v, part, valid, xq + (uint64_t)row * ldq + 32u * blk + 4u * part, xds + (uint64_t)row * nblk + blk);
     }
 }
 
@@ -99,9 +104,19 @@ RFXQ_DEV int act_f16_exp(float mx) {
 
 RFXQ_DEV float absmax4(float4 v) { return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))); }
 
-// the f16 layout of one row's four values at column c (lane's chunk)
+// The int8 layout beside the f16 one, from the same read of the values (I8):
+// [rows][k] and [rows][k/32]. Written by the producers whose buffers hold both.
+struct ActI8 {
+    int8_t* xq;
+    uint32_t* xds;
+};
+
+// the layouts of one row's four values at column c (lane's chunk)
+template <bool I8>
 RFXQ_DEV void act_f16_chunk(float4 v, uint32_t lane, uint32_t c, uint64_t ro, uint32_t r, uint32_t nsb, float scale,
-                            uint16_t* __restrict__ xh, uint16_t* __restrict__ xsx, float* __restrict__ yout) {
+                            uint16_t* __restrict__ xh, uint16_t* __restrict__ xsx, float* __restrict__ yout,
+                            const ActI8& i8) {
+    if constexpr (I8) q8_1_chunk(v, lane & 7u, true, i8.xq + ro + c, i8.xds + (ro + c) / 32u);
     if (yout) *reinterpret_cast<float4*>(yout + ro + c) = v;
     const half_t h0 = (half_t)(v.x * scale), h1 = (half_t)(v.y * scale);
     const half_t h2 = (half_t)(v.z * scale), h3 = (half_t)(v.w * scale);
@@ -140,8 +155,10 @@ RFXQ_DEV void act_f16_row_load(const Src& src, uint32_t r, uint32_t k, float4 (&
         if (i < nsb) v[i] = src.load(r, 4u * lane + 256u * i);
 }
 
+template <bool I8 = false>
 RFXQ_DEV void act_f16_row_put(const float4 (&v)[kActRowRegs], uint32_t r, uint32_t k, uint16_t* __restrict__ xh,
-                              uint16_t* __restrict__ xsx, float* __restrict__ xrs, float* __restrict__ yout) {
+                              uint16_t* __restrict__ xsx, float* __restrict__ xrs, float* __restrict__ yout,
+                              const ActI8& i8 = {}) {
     const uint32_t lane = threadIdx.x & 63u;
     const uint64_t ro = (uint64_t)r * k;
     const uint32_t nsb = k / 256u;
@@ -153,17 +170,18 @@ RFXQ_DEV void act_f16_row_put(const float4 (&v)[kActRowRegs], uint32_t r, uint32
     const float scale = ldexpf(1.0f, -e);
 #pragma unroll
     for (uint32_t i = 0; i < kActRowRegs; i++)
-        if (i < nsb) act_f16_chunk(v[i], lane, 4u * lane + 256u * i, ro, r, nsb, scale, xh, xsx, yout);
+        if (i < nsb) act_f16_chunk<I8>(v[i], lane, 4u * lane + 256u * i, ro, r, nsb, scale, xh, xsx, yout, i8);
     if (lane == 0u) xrs[r] = ldexpf(1.0f, e);
 }
 
-template <class Src>
+template <bool I8 = false, class Src>
 RFXQ_DEV void act_f16_row(const Src& src, uint32_t r, uint32_t k, uint16_t* __restrict__ xh,
-                          uint16_t* __restrict__ xsx, float* __restrict__ xrs, float* __restrict__ yout) {
+                          uint16_t* __restrict__ xsx, float* __restrict__ xrs, float* __restrict__ yout,
+                          const ActI8& i8 = {}) {
     if (k <= kActRegK) {
         float4 v[kActRowRegs];
         act_f16_row_load(src, r, k, v);
-        act_f16_row_put(v, r, k, xh, xsx, xrs, yout);
+        act_f16_row_put<I8>(v, r, k, xh, xsx, xrs, yout, i8);
         return;
     }
     const uint32_t lane = threadIdx.x & 63u;
@@ -173,74 +191,63 @@ RFXQ_DEV void act_f16_row(const Src& src, uint32_t r, uint32_t k, uint16_t* __re
     for (uint32_t c = 4u * lane; c < k; c += 256u) mx = fmaxf(mx, absmax4(src.load(r, c)));
     const int e = act_f16_exp(mx);
     const float scale = ldexpf(1.0f, -e);
-    for (uint32_t c = 4u * lane; c < k; c += 256u) act_f16_chunk(src.load(r, c), lane, c, ro, r, nsb, scale, xh, xsx, yout);
+    for (uint32_t c = 4u * lane; c < k; c += 256u)
+        act_f16_chunk<I8>(src.load(r, c), lane, c, ro, r, nsb, scale, xh, xsx, yout, i8);
     if (lane == 0u) xrs[r] = ldexpf(1.0f, e);
 }
 
-// One row by the whole 256-thread workgroup: thread t takes the four values
-// at 4t + 1024i, held in registers up to 16384 values (longer rows are read
-// twice); the row maximum
-// combines the four waves through LDS. Same layouts and arithmetic as
-// act_f16_row (the block sums are formed by the same 8 lanes in the same
-// order), so the result does not depend on which form wrote it.
-template <class Src>
+// One row by a whole workgroup of NT threads: thread t takes the four values
+// at 4t + 4 NT i, held in registers up to 16384 values (longer rows are read
+// twice); the row maximum combines the waves through LDS. Same layouts and
+// arithmetic as act_f16_row (the block sums are formed by the same 8 lanes in
+// the same order), so the result does not depend on which form wrote it.
+// NT = 1024 keeps four float4 a thread, and so all of a CU's waves resident
+// (256 threads with 16 float4 each: 64-79 us for both layouts of 2048 rows of
+// 14336, bound by the loads in flight).
+template <bool I8 = false, uint32_t NT = 256, class Src>
 RFXQ_DEV void act_f16_row_wg(const Src& src, uint32_t r, uint32_t k, uint16_t* __restrict__ xh,
-                             uint16_t* __restrict__ xsx, float* __restrict__ xrs, float* __restrict__ yout) {
-    __shared__ float wmax[4];
+                             uint16_t* __restrict__ xsx, float* __restrict__ xrs, float* __restrict__ yout,
+                             const ActI8& i8 = {}) {
+    __shared__ float wmax[NT / 64u];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint64_t ro = (uint64_t)r * k;
     const uint32_t nsb = k / 256u;
-    constexpr uint32_t NC = 16;  // rows up to 16384 values stay in registers
+    constexpr uint32_t NC = 16384u / (4u * NT);  // rows up to 16384 values stay in registers
     float4 v[NC];
     float mx = 0.0f;
-    const bool reg = k <= NC * 1024u;
+    const bool reg = k <= 16384u;
     if (reg) {
 #pragma unroll
         for (uint32_t i = 0; i < NC; i++) {
-            const uint32_t c = 4u * tid + 1024u * i;
+            const uint32_t c = 4u * tid + 4u * NT * i;
             if (c < k) v[i] = src.load(r, c);
         }
 #pragma unroll
         for (uint32_t i = 0; i < NC; i++)
-            if (4u * tid + 1024u * i < k) mx = fmaxf(mx, absmax4(v[i]));
+            if (4u * tid + 4u * NT * i < k) mx = fmaxf(mx, absmax4(v[i]));
     } else {
-        for (uint32_t c = 4u * tid; c < k; c += 1024u) mx = fmaxf(mx, absmax4(src.load(r, c)));
+        for (uint32_t c = 4u * tid; c < k; c += 4u * NT) mx = fmaxf(mx, absmax4(src.load(r, c)));
     }
     mx = wave_max(mx);
     if (lane == 0u) wmax[tid >> 6] = mx;
     __syncthreads();
-    mx = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+    mx = 0.0f;
+#pragma unroll
+    for (uint32_t i = 0; i < NT / 64u; i++) mx = fmaxf(mx, wmax[i]);
     __syncthreads();  // wmax is reused by the next row
     const int e = act_f16_exp(mx);
     const float scale = ldexpf(1.0f, -e);
     if (reg) {
 #pragma unroll
         for (uint32_t i = 0; i < NC; i++) {
-            const uint32_t c = 4u * tid + 1024u * i;
-            if (c < k) act_f16_chunk(v[i], lane, c, ro, r, nsb, scale, xh, xsx, yout);
+            const uint32_t c = 4u * tid + 4u * NT * i;
+            if (c < k) act_f16_chunk<I8>(v[i], lane, c, ro, r, nsb, scale, xh, xsx, yout, i8);
         }
     } else {
-        for (uint32_t c = 4u * tid; c < k; c += 1024u) act_f16_chunk(src.load(r, c), lane, c, ro, r, nsb, scale, xh, xsx, yout);
+        for (uint32_t c = 4u * tid; c < k; c += 4u * NT)
+            act_f16_chunk<I8>(src.load(r, c), lane, c, ro, r, nsb, scale, xh, xsx, yout, i8);
     }
     if (tid == 0u) xrs[r] = ldexpf(1.0f, e);
-}
-
-// Rows per workgroup of the f16 activation kernels: a row per wave (4 per
-// workgroup) for many short rows, a whole workgroup per row otherwise (few
-// rows, or rows too long for one wave's registers). The host sizes grids by
-// the same rule.
-RFXQ_DEV bool act_wave_rows(uint32_t rows, uint32_t k) { return k <= kActRegK && rows >= 128u; }
-
-template <class Src>
-RFXQ_DEV void act_f16_rows(const Src& src, uint32_t rows, uint32_t k, uint32_t b, uint32_t nb,
-                           uint16_t* __restrict__ xh, uint16_t* __restrict__ xsx, float* __restrict__ xrs,
-                           float* __restrict__ yout) {
-    if (act_wave_rows(rows, k)) {
-        for (uint32_t r = b * 4u + (threadIdx.x >> 6); r < rows; r += nb * 4u)
-            act_f16_row(src, r, k, xh, xsx, xrs, yout);
-    } else {
-        for (uint32_t r = b; r < rows; r += nb) act_f16_row_wg(src, r, k, xh, xsx, xrs, yout);
-    }
 }
 
 extern "C" __global__ __launch_bounds__(256) void rfxq_act_f16(const float* __restrict__ x, uint32_t ldx,
@@ -252,14 +259,38 @@ extern "C" __global__ __launch_bounds__(256) void rfxq_act_f16(const float* __re
         act_f16_row(src, r, k, xh, xsx, xrs, nullptr);
 }
 
+constexpr uint32_t kActWgThreads = 1024;  // of the row-per-workgroup kernels (the host launches as many)
+
 // the same with a row per workgroup (few or long rows; a kernel of its own:
 // its registers would otherwise limit the row-per-wave kernel's occupancy)
-extern "C" __global__ __launch_bounds__(256) void rfxq_act_f16_wg(const float* __restrict__ x, uint32_t ldx,
+extern "C" __global__ __launch_bounds__(1024) void rfxq_act_f16_wg(const float* __restrict__ x, uint32_t ldx,
                                                                  const int32_t* __restrict__ src_rows, uint32_t rows,
                                                                  uint32_t k, uint16_t* __restrict__ xh,
                                                                  uint16_t* __restrict__ xsx, float* __restrict__ xrs) {
     const QuantSrcPlain src{x, ldx, src_rows};
-    for (uint32_t r = blockIdx.x; r < rows; r += gridDim.x) act_f16_row_wg(src, r, k, xh, xsx, xrs, nullptr);
+    for (uint32_t r = blockIdx.x; r < rows; r += gridDim.x) act_f16_row_wg<false, kActWgThreads>(src, r, k, xh, xsx, xrs, nullptr);
+}
+
+// Both layouts (a caller's activation buffer) from one read of x, a row per
+// wave or per workgroup as above: 2048 rows of 14336 take 45 us (212 MB,
+// 4.7 TB/s) against 30 + 34 us as one pass for each layout.
+extern "C" __global__ __launch_bounds__(256) void rfxq_act_both(const float* __restrict__ x, uint32_t rows, uint32_t k,
+                                                               int8_t* __restrict__ xq, uint32_t* __restrict__ xds,
+                                                               uint16_t* __restrict__ xh, uint16_t* __restrict__ xsx,
+                                                               float* __restrict__ xrs) {
+    const QuantSrcPlain src{x, k, nullptr};
+    for (uint32_t r = blockIdx.x * 4u + (threadIdx.x >> 6); r < rows; r += gridDim.x * 4u)
+        act_f16_row<true>(src, r, k, xh, xsx, xrs, nullptr, ActI8{xq, xds});
+}
+extern "C" __global__ __launch_bounds__(1024) void rfxq_act_both_wg(const float* __restrict__ x, uint32_t rows,
+                                                                  uint32_t k, int8_t* __restrict__ xq,
+                                                                  uint32_t* __restrict__ xds,
+                                                                  uint16_t* __restrict__ xh,
+                                                                  uint16_t* __restrict__ xsx,
+                                                                  float* __restrict__ xrs) {
+    const QuantSrcPlain src{x, k, nullptr};
+    for (uint32_t r = blockIdx.x; r < rows; r += gridDim.x)
+        act_f16_row_wg<true, kActWgThreads>(src, r, k, xh, xsx, xrs, nullptr, ActI8{xq, xds});
 }
 
 // Several activations in one launch (grouped GEMMs): workgroups
@@ -290,11 +321,12 @@ extern "C" __global__ __launch_bounds__(256) void rfxq_act_f16_multi(const ActF1
         act_f16_row(src, r, d.k, d.xh, d.xsx, d.xrs, nullptr);
 }
 
-extern "C" __global__ __launch_bounds__(256) void rfxq_act_f16_multi_wg(const ActF16Desc* __restrict__ table,
+extern "C" __global__ __launch_bounds__(1024) void rfxq_act_f16_multi_wg(const ActF16Desc* __restrict__ table,
                                                                        uint32_t ndesc) {
     const ActF16Desc d = act_f16_pick(table, ndesc);
     const QuantSrcPlain src{d.x, d.k, nullptr};
-    for (uint32_t r = blockIdx.x - d.wg_begin; r < d.rows; r += d.wgs) act_f16_row_wg(src, r, d.k, d.xh, d.xsx, d.xrs, nullptr);
+    for (uint32_t r = blockIdx.x - d.wg_begin; r < d.rows; r += d.wgs)
+        act_f16_row_wg<false, kActWgThreads>(src, r, d.k, d.xh, d.xsx, d.xrs, nullptr);
 }
 
 extern "C" __global__ __launch_bounds__(256) void rfxq_quantize_q8_1(const float* __restrict__ x, uint32_t ldx,
@@ -387,15 +419,29 @@ extern "C" __global__ __launch_bounds__(256) void rfxq_rmsnorm_q8_1(const float*
         if (tid >= 64u) {
             if (c + 1u < nchunks) copy(c + 1u, tid - 64u, 192u);
         } else if (tid < nr) {
+            // eight values' reads a step ahead of their multiply-adds, so that
+            // the chain itself is the bound (len4 is a multiple of 64)
             const float4* sr = &stage[c & 1u][tid * kRowF4];
             const uint32_t len4 = min(kNormChunk, k - c * kNormChunk) / 4u;
-#pragma unroll 8
-            for (uint32_t j = 0; j < len4; j++) {
-                const float4 v = sr[j];
-                sum_sq = __builtin_fmaf(v.x, v.x, sum_sq);
-                sum_sq = __builtin_fmaf(v.y, v.y, sum_sq);
-                sum_sq = __builtin_fmaf(v.z, v.z, sum_sq);
-                sum_sq = __builtin_fmaf(v.w, v.w, sum_sq);
+            float4 v[2][8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) v[0][u] = sr[u];
+            for (uint32_t j = 0; j < len4; j += 16u) {
+#pragma unroll
+                for (int hf = 0; hf < 2; hf++) {
+                    const uint32_t nx = min(j + 8u * hf + 8u, len4 - 8u);
+#pragma unroll
+                    for (int u = 0; u < 8; u++) v[hf ^ 1][u] = sr[nx + u];
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int u = 0; u < 8; u++) {
+                        sum_sq = __builtin_fmaf(v[hf][u].x, v[hf][u].x, sum_sq);
+                        sum_sq = __builtin_fmaf(v[hf][u].y, v[hf][u].y, sum_sq);
+                        sum_sq = __builtin_fmaf(v[hf][u].z, v[hf][u].z, sum_sq);
+                        sum_sq = __builtin_fmaf(v[hf][u].w, v[hf][u].w, sum_sq);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
         }
         __syncthreads();
@@ -404,12 +450,11 @@ extern "C" __global__ __launch_bounds__(256) void rfxq_rmsnorm_q8_1(const float*
     __syncthreads();
     const uint64_t o = (uint64_t)r0 * k, nblk = k / 32u;
     const QuantSrcRms src{x + o, g, rinv, k};
-    // int8 layout (8 lanes per 32-block), then the f16 layout (one wave per
-    // row); the producer's own output y is written by the first pass run
-    if (xq) quant_q8_1_rows(src, nr, k, xq + o, k, xds + r0 * nblk, y ? y + o : nullptr, threadIdx.x >> 6, 4u);
+    // both layouts and y, one wave per row
     const uint32_t wv = threadIdx.x >> 6;
-    if (xh && wv < nr)
-        act_f16_row(src, wv, k, xh + o, xsx + r0 * (nblk / 8u) * 16u, xrs + r0, (!xq && y) ? y + o : nullptr);
+    if (wv < nr)
+        act_f16_row<true>(src, wv, k, xh + o, xsx + r0 * (nblk / 8u) * 16u, xrs + r0, y ? y + o : nullptr,
+                          ActI8{xq + o, xds + r0 * nblk});
 }
 
 // SiLU(gate) * up (src/kernels_cuda/silu_and_mul.cu:7-23: g / (1 + expf(-g)) * u)
@@ -426,7 +471,7 @@ struct QuantSrcSilu {
     }
 };
 
-extern "C" __global__ __launch_bounds__(256) void rfxq_silu_and_mul_q8_1(const float* __restrict__ gate,
+extern "C" __global__ __launch_bounds__(1024) void rfxq_silu_and_mul_q8_1(const float* __restrict__ gate,
                                                                         const float* __restrict__ up,
                                                                         uint32_t rows, uint32_t k,
                                                                         int8_t* __restrict__ xq,
@@ -436,8 +481,11 @@ extern "C" __global__ __launch_bounds__(256) void rfxq_silu_and_mul_q8_1(const f
                                                                         float* __restrict__ xrs,
                                                                         float* __restrict__ y) {
     const QuantSrcSilu src{gate, up, k};
-    if (xq)
+    for (uint32_t r = blockIdx.x; r < rows && xh; r += gridDim.x) {
+        if (xq) act_f16_row_wg<true, kActWgThreads>(src, r, k, xh, xsx, xrs, y, ActI8{xq, xds});
+        else act_f16_row_wg<false, kActWgThreads>(src, r, k, xh, xsx, xrs, y);
+    }
+    if (!xh && xq)
         quant_q8_1_rows(src, rows, k, xq, k, xds, y, ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6,
                         ((uint64_t)gridDim.x * blockDim.x) >> 6);
-    if (xh) act_f16_rows(src, rows, k, blockIdx.x, gridDim.x, xh, xsx, xrs, xq ? nullptr : y);
 }

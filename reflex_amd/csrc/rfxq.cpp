@@ -154,6 +154,7 @@ struct Ctx {
     hipFunction_t mmqh_mix_m32 = nullptr;  // 32-row tiles, Q4_K or Q6_K per descriptor
     hipFunction_t mmqs = nullptr;          // up to 32 rows, any type per descriptor
     hipFunction_t mmqh_n128 = nullptr;     // 64 x 128 tiles, any type per descriptor
+    hipFunction_t act_both = nullptr, act_both_wg = nullptr;  // both layouts from one read
     hipFunction_t act_f16 = nullptr, act_f16_multi = nullptr, act_f16_wg = nullptr, act_f16_multi_wg = nullptr;
     hipFunction_t deq[3][2] = {};
     hipFunction_t gather = nullptr, scatter = nullptr, silu = nullptr, combine = nullptr;
@@ -233,6 +234,8 @@ int load_ctx(int device, Ctx** out) {
         {&c->mmqh_mix_m32, "rfxq_mmqh_mix_m32"},
         {&c->mmqs, "rfxq_mmqs"},
         {&c->mmqh_n128, "rfxq_mmqh_n128"},
+        {&c->act_both, "rfxq_act_both"},
+        {&c->act_both_wg, "rfxq_act_both_wg"},
         {&c->act_f16, "rfxq_act_f16"},
         {&c->act_f16_multi, "rfxq_act_f16_multi"},
         {&c->act_f16_wg, "rfxq_act_f16_wg"},
@@ -1128,6 +1131,7 @@ int launch_quant(Ctx* c, const float* x, uint32_t ldx, const int32_t* src_rows, 
 // workgroup (rfxq_act_f16[_multi]_wg: few rows, or rows too long for one
 // wave's registers)
 bool act_f16_wave(uint32_t rows, uint32_t k) { return k <= 4096u && rows >= 128u; }
+constexpr uint32_t kActWgThreads = 1024;  // of the row-per-workgroup kernels (quant.hpp)
 uint32_t act_f16_grid(uint32_t rows, bool wave) {
     return wave ? std::min<uint32_t>((rows + 3u) / 4u, 4096u) : std::min<uint32_t>(rows, 16384u);
 }
@@ -1148,12 +1152,28 @@ int launch_act_f16(Ctx* c, const float* x, uint32_t ldx, const int32_t* src_rows
     // chip; 512 rows of 2048 take 6 us as 512 workgroups against 9.6 us as 128)
     const bool wave = act_f16_wave(rows, k) && rows >= 1024u;
     return launch(wave ? c->act_f16 : c->act_f16_wg, act_f16_grid(rows, wave), 0, stream, &a, sizeof a,
-                  "rfxq_act_f16 launch");
+                  "rfxq_act_f16 launch", wave ? 256u : kActWgThreads);
 }
 
 // the activation layouts of L at `base` from x
 int launch_act(Ctx* c, const float* x, uint32_t rows, uint32_t k, uint8_t* base, const ActLayout& L, bool i8,
                bool h, hipStream_t stream) {
+    if (i8 && h) {
+        struct {
+            const float* x;
+            uint32_t rows, k;
+            int8_t* xq;
+            uint32_t* xds;
+            uint16_t* xh;
+            uint16_t* xsx;
+            float* xrs;
+        } a = {x, rows, k, reinterpret_cast<int8_t*>(base + L.xq), reinterpret_cast<uint32_t*>(base + L.xds),
+               reinterpret_cast<uint16_t*>(base + L.xh), reinterpret_cast<uint16_t*>(base + L.xsx),
+               reinterpret_cast<float*>(base + L.xrs)};
+        const bool wave = act_f16_wave(rows, k) && rows >= 1024u;  // as launch_act_f16
+        return launch(wave ? c->act_both : c->act_both_wg, act_f16_grid(rows, wave), 0, stream, &a, sizeof a,
+                      "rfxq_act_both launch", wave ? 256u : kActWgThreads);
+    }
     if (i8)
         if (int rc = launch_quant(c, x, k, nullptr, rows, k, reinterpret_cast<int8_t*>(base + L.xq),
                                   reinterpret_cast<uint32_t*>(base + L.xds), stream))
@@ -1188,8 +1208,8 @@ int launch_silu_act(Ctx* c, const float* gate, const float* up, uint32_t rows, u
            h ? reinterpret_cast<uint16_t*>(base + L.xsx) : nullptr,
            h ? reinterpret_cast<float*>(base + L.xrs) : nullptr,
            nullptr};
-    const uint32_t grid = i8 ? quant_grid((uint64_t)rows * (k / 32u)) : act_f16_grid(rows, act_f16_wave(rows, k));
-    return launch(c->silu_q, grid, 0, stream, &a, sizeof a, "rfxq_silu_and_mul_q8_1 launch");
+    const uint32_t grid = h ? act_f16_grid(rows, false) : (quant_grid((uint64_t)rows * (k / 32u)) + 3u) / 4u;
+    return launch(c->silu_q, grid, 0, stream, &a, sizeof a, "rfxq_silu_and_mul_q8_1 launch", kActWgThreads);
 }
 
 // rfxq_moe_combine: out[t,:] = sum over the token's k pairs of w * pair_out row
@@ -2210,8 +2230,8 @@ int rfxq_silu_and_mul_q8_1(const float* gate, const float* up, uint32_t rows, ui
     } a = {gate, up, rows, k, reinterpret_cast<int8_t*>(b + L.xq), reinterpret_cast<uint32_t*>(b + L.xds),
            reinterpret_cast<uint16_t*>(b + L.xh), reinterpret_cast<uint16_t*>(b + L.xsx),
            reinterpret_cast<float*>(b + L.xrs), y};
-    if (int rc = launch(c->silu_q, quant_grid((uint64_t)rows * (k / 32u)), 0, stream, &a, sizeof a,
-                        "rfxq_silu_and_mul_q8_1 launch"))
+    if (int rc = launch(c->silu_q, act_f16_grid(rows, false), 0, stream, &a, sizeof a, "rfxq_silu_and_mul_q8_1 launch",
+                        kActWgThreads))
         return rc;
     return ok();
 }
@@ -2492,7 +2512,7 @@ int rfxq_gemm_plan_run(const rfxq_gemm_plan* plan, hipStream_t stream) {
             uint32_t ndesc, pad;
         } ha = {plan->htable, plan->nh, 0};
         if (int rc = launch(plan->hwave ? c->act_f16_multi : c->act_f16_multi_wg, plan->hgrid, 0, stream, &ha, sizeof ha,
-                            "rfxq_act_f16_multi launch"))
+                            "rfxq_act_f16_multi launch", plan->hwave ? 256u : kActWgThreads))
             return rc;
     }
     for (uint32_t t = 0; t < kGroupKernels; t++) {
