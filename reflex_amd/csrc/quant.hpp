@@ -272,8 +272,8 @@ extern "C" __global__ __launch_bounds__(1024) void rfxq_act_f16_wg(const float* 
 }
 
 // Both layouts (a caller's activation buffer) from one read of x, a row per
-// wave or per workgroup as above: 2048 rows of 14336 take 45 us (212 MB,
-// 4.7 TB/s) against 30 + 34 us as one pass for each layout.
+// wave or per workgroup as above: 2048 rows of 14336 take 53 us (212 MB,
+// 4.0 TB/s) against 30 + 34 us as one pass for each layout.
 extern "C" __global__ __launch_bounds__(256) void rfxq_act_both(const float* __restrict__ x, uint32_t rows, uint32_t k,
                                                                int8_t* __restrict__ xq, uint32_t* __restrict__ xds,
                                                                uint16_t* __restrict__ xh, uint16_t* __restrict__ xsx,
