@@ -176,7 +176,8 @@ void rfxq_gemv_plan_destroy(rfxq_gemv_plan* plan);
  * = d_bits | s_bits << 16 (d = amax/127, q = roundf(x/d), s = d*sum(q)). */
 int rfxq_quantize_q8_1(const float* x, uint32_t rows, uint32_t k, int8_t* xq, uint32_t* xds, hipStream_t stream);
 
-/* Bytes of workspace rfxq_gemm needs for this weight and row count. */
+/* Bytes of workspace rfxq_gemm needs for this weight and row count (an output
+ * over the input included). */
 uint64_t rfxq_gemm_workspace_size(const rfxq_weight* w, uint32_t rows);
 
 /* Model::gemm (src/model/kernels.rs:2197) on a quantized-resident weight:

@@ -914,6 +914,25 @@ uint32_t few_max_sb(uint32_t rows) { return rows > 32u ? 0u : rows > 16u ? 4u : 
 uint32_t few_lds(uint32_t rows, uint32_t sb) {
     return 128u + std::max(16384u, rows * (sb * 544u + 16u));  // (results pass through 4 KB per wave)
 }
+// Whether one launch of `tiles` 32 x 256 tiles (`load` super-blocks over all
+// of them, the longest row max_nsb) runs on the few-row kernel. It keeps more
+// weight bytes in flight than the 32-row tiles, but each of its workgroups
+// brings the f32 rows in itself, and its short ranges write more partials:
+// both grow with the rows, and the tiles catch up once they fill the CUs.
+// Measured, 32-row tiles -> few-row kernel (us), Q4_K / Q6_K / Q8_0:
+//   4096 x 4096       16 rows 15 -> 12 / 18 -> 16 / 17 -> 15;   32: 17 -> 15 / 19 -> 18 / 19 -> 18
+//   32768 x 2048      16 rows 25 -> 20 / 37 -> 26 / 44 -> 31;   32: 26 -> 25 / 37 -> 30 / 45 -> 34
+//   8B layer (3300 super-blocks of tiles)  24 rows 78 -> 74, Q8_0 90 -> 88;  32: 78 -> 79, 91 -> 93
+//   65536 x 1024      16 rows 18 -> 23 / 26 -> 28 / 26 -> 32;   32: 19 -> 30 / 26 -> 35 / 26 -> 37
+//   65536 x 2048       8 rows 29 -> 26 / 41 -> 38 / 46 -> 43;   16: 29 -> 31 / 41 -> 41 / 46 -> 46
+//   65536 x 4096      16 rows 50 -> 47 / 75 -> 71 / 104 -> 92;  32: 48 -> 61 / 76 -> 82 / 106 -> 107
+//   128256 x 4096      8 rows 86 -> 79 / 167 -> 131 / 208 -> 180;   16: 85 -> 88 / 169 -> 140 / 209 -> 188
+//   151936 x 1024     16 rows 34 -> 33 / 62 -> 49 / 64 -> 53;   32: 35 -> 40 / 64 -> 54 / 66 -> 59
+bool few_wins(uint32_t tiles, uint64_t load, uint32_t max_nsb, uint32_t rows, bool q4k, uint32_t cus) {
+    if (tiles < cus) return rows <= 24u || load <= 8ull * cus;
+    if (rows <= (q4k ? 8u : 16u)) return max_nsb > 4u || tiles >= 2u * cus;
+    return !q4k && max_nsb <= 4u && tiles >= 2u * cus;  // (one range: no partials)
+}
 
 // Row tile of one grouped MoE GEMM, `pairs` routed rows over `experts`
 // groups, `tiles_n` column tiles per expert: f16 kernels 32-row tiles up to
@@ -1043,13 +1062,10 @@ rfxq_gemm_policy gemm_policy(uint32_t ty, uint32_t k, uint32_t n, uint32_t rows,
     if (f16 && alone && !o.quant_mma_splits && rows >= 256u) p.tile_m = small_gemm_tile_m(p.tile_m, rows, n, nsb, cus);
     const uint32_t tiles = ((rows + p.tile_m - 1u) / p.tile_m) * ((n + p.tile_n - 1u) / p.tile_n);
     uint32_t splits = 1;
-    const uint32_t few = f16 ? few_max_sb(rows) : 0u;
     if (o.quant_mma_splits) splits = o.quant_mma_splits;
-    else if (2u * tiles < std::max(cus, 1u) || few) {
-        // 32-row tiles stream weights (few rows): splits down to one
-        // super-block, and ranges that the few-row kernel can hold
-        uint32_t w = split_sb({{tiles, nsb}}, p.tile_m == 32u ? 1u : 2u, 2u * std::max(cus, 1u));
-        if (few) w = std::min(w, few);
+    else if (2u * tiles < std::max(cus, 1u)) {
+        // 32-row tiles stream weights (few rows): splits down to one super-block
+        const uint32_t w = split_sb({{tiles, nsb}}, p.tile_m == 32u ? 1u : 2u, 2u * std::max(cus, 1u));
         splits = (nsb + w - 1u) / w;
     }
     splits = std::min(std::max(1u, splits), nsb);
@@ -1297,30 +1313,59 @@ struct GemmPlan {
 };
 
 // an MMQ plan for a GEMM the policy sends to an MMQ path
-// (`in_place`: y overlaps x, which must then be read before any result is written)
-GemmPlan plan_gemm(const Ctx* c, const rfxq_weight* w, uint32_t rows, const rfxq_options& o, bool in_place = false) {
+// (`in_place`: y overlaps x, which must then be read before any result is
+// written; `general`: the policy's own tiles and splits, where the workspace
+// that the others need is not there)
+GemmPlan plan_gemm(const Ctx* c, const rfxq_weight* w, uint32_t rows, const rfxq_options& o, bool in_place = false,
+                   bool general = false) {
     GemmPlan p;
-    const uint32_t k = w->in_features, n = w->out_features;
-    p.pol = gemm_policy(w->ggml_type, k, n, rows, c ? (uint32_t)c->cus : 256u, o);
+    const uint32_t k = w->in_features, n = w->out_features, nsb = k / 256u;
+    const uint32_t cus = c ? (uint32_t)c->cus : 256u;
+    p.pol = gemm_policy(w->ggml_type, k, n, rows, cus, o);
     p.f16 = p.pol.path == PATH_MMQ_F16;
     if (p.pol.path == PATH_GEMV_ROWS) return p;  // no MMQ launch: tiles, layouts and workspace stay 0
-    const uint32_t cus = c ? (uint32_t)c->cus : 256u;
-    if (uint32_t sb = p.f16 && !o.quant_mma_splits ? n128_sb({{n, k / 256u}}, w->ggml_type, rows, cus,
-                                                             {p.pol.tile_m, p.pol.sb_per_split})
-                                                   : 0u) {
-        p.n128 = true;
-        p.pol.tile_m = 64u;
-        p.pol.tile_n = 128u;
-        p.pol.sb_per_split = sb;
-        p.pol.splits = (k / 256u + sb - 1u) / sb;
+    const bool forced = o.quant_mma_splits != 0;
+    uint32_t sb = 0;
+    if (p.f16 && !general && !in_place && few_max_sb(rows)) {
+        const uint32_t tiles = (n + 255u) / 256u;
+        if (forced) p.few = p.pol.sb_per_split <= few_max_sb(rows);
+        else if (few_wins(tiles, (uint64_t)tiles * nsb, nsb, rows, w->ggml_type == RFXQ_TYPE_Q4_K, cus)) {
+            p.few = true;
+            sb = std::min(split_sb({{tiles, nsb}}, 1u, 2u * std::max(cus, 1u)), few_max_sb(rows));
+        }
+    } else if (p.f16 && !general && !forced) {
+        sb = n128_sb({{n, nsb}}, w->ggml_type, rows, cus, {p.pol.tile_m, p.pol.sb_per_split});
+        if (sb) {
+            p.n128 = true;
+            p.pol.tile_m = 64u;
+            p.pol.tile_n = 128u;
+        }
+    }
+    if (sb) {
+        p.pol.splits = (nsb + sb - 1u) / sb;
+        p.pol.sb_per_split = p.few ? (nsb + p.pol.splits - 1u) / p.pol.splits : sb;
     }
     p.tiles_m = (rows + p.pol.tile_m - 1u) / p.pol.tile_m;
     p.tiles_n = (n + p.pol.tile_n - 1u) / p.pol.tile_n;
-    p.few = p.f16 && !in_place && p.pol.sb_per_split <= few_max_sb(rows);
     if (!p.few) p.act = act_layout_sel(rows, k, !p.f16, p.f16);
     p.off_part = p.act.total;
     p.total = p.off_part + (p.pol.splits > 1 ? align256((uint64_t)p.pol.splits * rows * n * 4u) : 0u);
+    // more partials than the fixed scratch holds: the policy's plan if that
+    // needs less (one rule for every entry point, so that all give one result)
+    if (sb && p.total > rfxq_scratch::kScratchBytes) {
+        const GemmPlan g = plan_gemm(c, w, rows, o, in_place, true);
+        if (g.total < p.total) return g;
+    }
     return p;
+}
+
+// whether the library workspace holds `bytes` or can grow to them now
+bool ws_available(Ctx* c, uint64_t bytes, hipStream_t stream) {
+    {
+        std::lock_guard<std::mutex> lk(c->mu);
+        if (bytes <= c->ws_bytes) return true;
+    }
+    return !capturing(stream);
 }
 
 int launch_reduce(Ctx* c, const float* part, float* y, uint64_t n, uint32_t splits, hipStream_t stream) {
@@ -1367,7 +1412,9 @@ int gemm_run(Ctx* c, const GemmPlan& p, const float* x, const uint8_t* act, cons
 int gemm_impl(Ctx* c, const float* x, const rfxq_weight* w, uint32_t rows, float* y, void* ws, uint64_t ws_bytes,
               const rfxq_options& o, hipStream_t stream) {
     const bool in_place = overlap(x, 4ull * rows * w->in_features, y, 4ull * rows * w->out_features);
-    const GemmPlan p = plan_gemm(c, w, rows, o, in_place);
+    GemmPlan p = plan_gemm(c, w, rows, o, in_place);
+    if (p.total && (ws ? ws_bytes < p.total : !ws_available(c, p.total, stream)))
+        p = plan_gemm(c, w, rows, o, in_place, true);
     if (!ws) {
         if (int rc = ctx_workspace(c, p.total, &ws, stream)) return rc;
     } else if (ws_bytes < p.total) {
@@ -1445,8 +1492,9 @@ uint32_t group_index(uint32_t ty, bool f16, uint32_t tile_m) {
 // `ext` (optional, one per item): the items' x are caller activation buffers
 // (rfxq_act_q8_1_size layouts, already quantized): every GEMM takes an MMQ
 // kernel (f16 unless REFLEX_MMQ_F16=0) and the group quantizes nothing.
+// `general`: no few-row kernel and no 64 x 128 tiles (as in plan_gemm).
 int build_gemm_group(const rfxq_gemm_item* items, uint32_t count, uint32_t rows, GemmGroup* g, uint32_t cus,
-                     bool ext = false) {
+                     bool ext = false, bool general = false) {
     if (!items || count == 0 || rows == 0) return fail(RFXQ_ERR_INVALID_INPUT, "gemm group: empty");
     rfxq_options o;
     if (int rc = get_options(&o)) return rc;
@@ -1456,7 +1504,7 @@ int build_gemm_group(const rfxq_gemm_item* items, uint32_t count, uint32_t rows,
         if (items[i].w) group_bytes += gemm_weight_bytes(items[i].w->ggml_type, items[i].w->in_features, items[i].w->out_features);
     // the few-row kernel reads f32 activations while results are written: not
     // for a group with an output on one of its inputs
-    bool in_place = false;
+    bool in_place = general;
     for (uint32_t i = 0; i < count && few_max_sb(rows) && !ext; i++)
         for (uint32_t j = 0; j < count && items[i].w; j++)
             in_place |= items[j].w && overlap(items[i].x, 4ull * rows * items[i].w->in_features, items[j].y,
@@ -1498,12 +1546,29 @@ int build_gemm_group(const rfxq_gemm_item* items, uint32_t count, uint32_t rows,
             return fail(RFXQ_ERR_OTHER, "gemm group: one x used with in_features %u and %u", g->acts[ai].k, k);
         }
         item_act[i] = (uint32_t)ai;
-        if (f16) g->acts[ai].need_h |= !few;
-        else g->acts[ai].need_i8 = true;
+        if (!f16) g->acts[ai].need_i8 = true;
+    }
+    // the few-row kernel, or tiles, for all its GEMMs (few_wins)
+    uint32_t few_tiles = 0, few_nsb = 0;
+    uint64_t few_load = 0;
+    bool few_q4k = false;
+    for (uint32_t i = 0; i < count; i++) {
+        if (item_act[i] == ~0u || item_kernel[i] != kGroupFew) continue;
+        const uint32_t tiles = (items[i].w->out_features + 255u) / 256u, nsb = items[i].w->in_features / 256u;
+        few_tiles += tiles;
+        few_load += (uint64_t)tiles * nsb;
+        few_nsb = std::max(few_nsb, nsb);
+        few_q4k |= items[i].w->ggml_type == RFXQ_TYPE_Q4_K;
+    }
+    const bool few_kept = o.quant_mma_splits || few_wins(few_tiles, few_load, few_nsb, rows, few_q4k, cus);
+    for (uint32_t i = 0; i < count; i++) {
+        if (item_act[i] == ~0u) continue;
+        if (item_kernel[i] == kGroupFew && !few_kept) item_kernel[i] = group_index(items[i].w->ggml_type, true, 32u);
+        if (group_f16(item_kernel[i])) g->acts[item_act[i]].need_h |= item_kernel[i] != kGroupFew;
     }
     // the GEMMs of a type that 64 x 128 tiles are estimated to run faster
     // than the launch's larger tiles (split as below)
-    for (uint32_t t = 6u; t < kGroupFew && !o.quant_mma_splits; t++) {
+    for (uint32_t t = 6u; t < kGroupFew && !o.quant_mma_splits && !general; t++) {
         std::vector<GemmShape> shapes;
         std::vector<std::pair<uint32_t, uint32_t>> tn;
         uint32_t ty = 0, tiles = 0, max_nsb = 0;
@@ -2051,8 +2116,9 @@ uint64_t rfxq_gemm_workspace_size(const rfxq_weight* w, uint32_t rows) {
         if (it != g_ctx.end()) c = it->second.get();
     }
     if (!options_ok()) return 0;
-    const GemmPlan p = plan_gemm(c, w, rows, opt());
-    return p.pol.path == PATH_GEMV_ROWS ? 0 : p.total;
+    // with an output over its input too (both layouts are never held at once)
+    const GemmPlan p = plan_gemm(c, w, rows, opt()), q = plan_gemm(c, w, rows, opt(), true);
+    return p.pol.path == PATH_GEMV_ROWS ? 0 : std::max(p.total, q.total);
 }
 
 int rfxq_gemm(const float* x, uint64_t x_len, const rfxq_weight* w, uint32_t rows, float* y, void* workspace,
@@ -2117,7 +2183,7 @@ int rfxq_gemm_no_alloc(const float* x, uint64_t x_len, const rfxq_weight* w, uin
     }
     if (int rc = check_mmq_weight(w, "gemm_no_alloc")) return rc;
     if (reinterpret_cast<uintptr_t>(x) % 16u) return fail(RFXQ_ERR_OTHER, "gemm_no_alloc: x is not 16-byte aligned");
-    const GemmPlan p = plan_gemm(c, w, rows, o);
+    const GemmPlan p = plan_gemm(c, w, rows, o, overlap(x, 4ull * rows * w->in_features, y, 4ull * rows * w->out_features));
     if (p.total > rfxq_scratch::kScratchBytes)
         return fail(RFXQ_ERR_INVALID_INPUT,
                     "gemm_no_alloc: rows=%u in_features=%u out_features=%u needs %llu bytes of scratch; the fixed "
@@ -2134,6 +2200,10 @@ int rfxq_gemm_batch(const rfxq_gemm_item* items, uint32_t count, uint32_t rows, 
     if (int rc = current_ctx(&c)) return rc;
     GemmGroup g;
     if (int rc = build_gemm_group(items, count, rows, &g, (uint32_t)c->cus)) return rc;
+    if (!ws_available(c, g.ws_bytes, stream)) {
+        g = GemmGroup();
+        if (int rc = build_gemm_group(items, count, rows, &g, (uint32_t)c->cus, false, true)) return rc;
+    }
     void* ws = nullptr;
     if (int rc = ctx_workspace(c, g.ws_bytes, &ws, stream)) return rc;
     bind_gemm_group(&g, static_cast<uint8_t*>(ws));
@@ -2253,10 +2323,13 @@ int rfxq_gemm_q8_1(const void* act, uint32_t rows, const rfxq_weight* w, float* 
         o.quant_mma_max_rows = 0;
     }
     // one row plans as two (same tiles): the policy sends single rows to the GEMV
-    const GemmPlan p = plan_gemm(c, w, std::max(rows, 2u), o);
+    GemmPlan p = plan_gemm(c, w, std::max(rows, 2u), o);
+    auto partials = [&] { return p.pol.splits > 1 ? (uint64_t)p.pol.splits * rows * n * 4u : 0u; };
+    if (workspace ? workspace_bytes < partials() : !ws_available(c, partials(), stream))
+        p = plan_gemm(c, w, std::max(rows, 2u), o, false, true);
     float* part = nullptr;
     if (p.pol.splits > 1) {
-        const uint64_t need = (uint64_t)p.pol.splits * rows * n * 4u;
+        const uint64_t need = partials();
         void* ws = workspace;
         if (!ws) {
             if (int rc = ctx_workspace(c, need, &ws, stream)) return rc;

@@ -22,7 +22,7 @@ import numpy as np
 import pytest
 import torch
 
-from reflex_amd import synth
+from reflex_amd import lib, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -327,6 +327,45 @@ def test_gemm_few_rows_kernel(rq, orc, ty, m, n, k):
         over = x.clone()
         got = rq.gemm(over, w, m, out=over)[:m * n].cpu().numpy().reshape(m, n)
         assert np.abs(got - y).max() <= 1e-5 * np.abs(y).max()
+
+
+@pytest.mark.parametrize("ty", [Q4K, Q6K, Q8_0])
+@pytest.mark.parametrize("m,n,k", [(8, 131072, 512), (9, 65280, 768), (32, 65536, 768), (17, 131328, 256)])
+def test_gemm_few_rows_many_tiles(rq, ty, m, n, k):
+    """Launches of about one and two tiles per CU, where the few-row kernel and the 32-row tiles change places:
+    columns agree with a narrow GEMM over the same weights (their sums differ in the order of the super-blocks
+    only: k / 256 partials, each within 2^-24 of the sum of magnitudes)."""
+    w_np = synth.weights(ty, 512, k, 960)
+    x = _dev(synth.activations(m * k, 961))
+    reps = (n + 511) // 512
+    wide = np.tile(w_np.reshape(512, -1), (reps, 1))[:n]
+    y = rq.gemm(x, _weight(rq, ty, wide.reshape(-1), n, k), m).reshape(m, n)
+    ref = rq.gemm(x, _weight(rq, ty, w_np, 512, k), m).reshape(m, 512)
+    ref = ref.repeat(1, reps)[:, :n]
+    assert float((y - ref).abs().max()) <= 1e-5 * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("ty", [Q4K, Q6K, Q8_0])
+def test_gemm_few_rows_workspaces(rq, ty):
+    """Workspaces that hold the 32-row tiles' plan: the advertised bytes with an output over its input; none for
+    an activation buffer of two rows, whose f32 form runs as GEMVs; both take the tiles."""
+    n, k, m = 600, 4864, 20
+    w = _weight(rq, ty, synth.weights(ty, n, k, 970), n, k)
+    x = _dev(synth.activations(m * k, 971))
+    ws = torch.empty(rq.gemm_workspace_size(w, m), dtype=torch.uint8, device=DEV)
+    want = rq.gemm(x, w, m, workspace=ws)
+    over = x.clone()
+    got = rq.gemm(over, w, m, workspace=ws, out=over)[:m * n]
+    assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max())
+    n, k, m = 33024, 2304, 2
+    w = _weight(rq, ty, np.tile(synth.weights(ty, 256, k, 972).reshape(256, -1), (n // 256, 1)).reshape(-1), n, k)
+    assert rq.gemm_workspace_size(w, m) == 0
+    act = rq.quantize_act_q8_1(_dev(synth.activations(m * k, 973)), m, k)
+    want = rq.gemm_q8_1(act, w, m)
+    got, ws = torch.empty_like(want), torch.empty(256, dtype=torch.uint8, device=DEV)
+    assert lib().rfxq_gemm_q8_1(act.data_ptr(), m, w.cref(), got.data_ptr(), ws.data_ptr(), 256,
+                                torch.cuda.current_stream().cuda_stream) == 0
+    assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max())
 
 
 @pytest.mark.parametrize("ty", [Q4K, Q6K, Q8_0])

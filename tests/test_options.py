@@ -190,6 +190,16 @@ def test_policy_tiles_and_splits(rq):
     assert pol(Q6K, 4096, 1024, 512, 256)["splits"] == 8
 
 
+@pytest.mark.parametrize("ty", [Q4K, Q6K, Q8_0])
+@pytest.mark.parametrize("n,k,rows", [(151936, 8192, 32), (65280, 24576, 24), (32768, 32768, 16), (128256, 16384, 16)])
+def test_workspace_of_few_rows_fits_the_scratch(rq, ty, n, k, rows):
+    """Few rows of a wide matrix: the partials of short ranges would pass 128 MiB (the fixed scratch)
+    where the policy's own plan needs the f16 layout only."""
+    import torch
+    w = rq.Weight(rq.GgmlType(ty), torch.empty(16, dtype=torch.uint8), [k, n])
+    assert 0 < rq.gemm_workspace_size(w, rows) <= 128 << 20
+
+
 def test_policy_errors(rq):
     with pytest.raises(rq.GgmlError):
         rq.gemm_policy(2, 1024, 1024, 512)
