@@ -489,3 +489,15 @@ extern "C" __global__ __launch_bounds__(1024) void rfxq_silu_and_mul_q8_1(const 
         quant_q8_1_rows(src, rows, k, xq, k, xds, y, ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6,
                         ((uint64_t)gridDim.x * blockDim.x) >> 6);
 }
+
+// the same with a row per wave (many short rows), the f16 layout at least
+extern "C" __global__ __launch_bounds__(256) void rfxq_silu_and_mul_q8_1_wave(
+    const float* __restrict__ gate, const float* __restrict__ up, uint32_t rows, uint32_t k, int8_t* __restrict__ xq,
+    uint32_t* __restrict__ xds, uint16_t* __restrict__ xh, uint16_t* __restrict__ xsx, float* __restrict__ xrs,
+    float* __restrict__ y) {
+    const QuantSrcSilu src{gate, up, k};
+    for (uint32_t r = blockIdx.x * 4u + (threadIdx.x >> 6); r < rows; r += gridDim.x * 4u) {
+        if (xq) act_f16_row<true>(src, r, k, xh, xsx, xrs, y, ActI8{xq, xds});
+        else act_f16_row<false>(src, r, k, xh, xsx, xrs, y);
+    }
+}

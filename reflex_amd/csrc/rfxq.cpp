@@ -158,7 +158,8 @@ struct Ctx {
     hipFunction_t act_f16 = nullptr, act_f16_multi = nullptr, act_f16_wg = nullptr, act_f16_multi_wg = nullptr;
     hipFunction_t deq[3][2] = {};
     hipFunction_t gather = nullptr, scatter = nullptr, silu = nullptr, combine = nullptr;
-    hipFunction_t rms_q = nullptr, silu_q = nullptr, moe_route = nullptr, moe_route_w = nullptr, moe_plan = nullptr;
+    hipFunction_t rms_q = nullptr, silu_q = nullptr, silu_q_wave = nullptr;
+    hipFunction_t moe_route = nullptr, moe_route_w = nullptr, moe_plan = nullptr;
     // MoE decode kernels: [Q4_K, Q6_K, Q8_0][4, 8, 16, 32 lanes per row]
     hipFunction_t moe_dec_gu[3][4] = {}, moe_dec_dn[3][4] = {};
     void* ws = nullptr;
@@ -251,6 +252,7 @@ int load_ctx(int device, Ctx** out) {
         {&c->silu, "rfxq_silu_and_mul"},
         {&c->rms_q, "rfxq_rmsnorm_q8_1"},
         {&c->silu_q, "rfxq_silu_and_mul_q8_1"},
+        {&c->silu_q_wave, "rfxq_silu_and_mul_q8_1_wave"},
         {&c->moe_route, "rfxq_moe_route"},
         {&c->moe_route_w, "rfxq_moe_route_w"},
         {&c->moe_plan, "rfxq_moe_plan"},
@@ -1012,17 +1014,28 @@ double mmqh_time(const std::vector<GemmShape>& g, uint32_t rows, uint32_t bm, ui
 struct TileSplit {
     uint32_t tile_m, sb;
 };
+// Ranges no longer than the launch's shortest row: each XCD takes contiguous
+// tiles, and a GEMM of longer ones would keep its XCD busy alone (a Q8_0 8B
+// layer, K = 4096 and 14336: 198 us at 64 rows, 120 on 64 x 256 tiles, now
+// 90). Up to 1.25x where that keeps a workgroup per CU (the layer's Q6_K v and
+// down projections at 128 rows: 133 us for the layer, 144 with one range more).
+uint32_t n128_split(const std::vector<std::pair<uint32_t, uint32_t>>& tiles_nsb, uint32_t cus) {
+    const uint32_t sb = split_sb(tiles_nsb, 1u, std::max(1u, cus));
+    uint32_t shortest = ~0u;
+    uint64_t wgs = 0;
+    for (const auto& t : tiles_nsb) {
+        shortest = std::min(shortest, t.second);
+        wgs += (uint64_t)t.first * ((t.second + sb - 1u) / sb);
+    }
+    return wgs <= cus && 4u * sb <= 5u * shortest ? sb : std::min(sb, shortest);
+}
 uint32_t n128_sb(const std::vector<GemmShape>& g, uint32_t ty, uint32_t rows, uint32_t cus, TileSplit base) {
     static const double kBig[3] = {4.1, 5.5, 7.5}, kMid[3] = {2.9, 4.0, 4.5}, kSmall[3] = {1.65, 2.35, 2.5};
     if (rows <= 32u) return 0u;
     const int t = type_index(ty);
     std::vector<std::pair<uint32_t, uint32_t>> tiles;
-    uint32_t max_nsb = 1;
-    for (const auto& s : g) {
-        tiles.push_back({((rows + 63u) / 64u) * ((s.n + 127u) / 128u), s.nsb});
-        max_nsb = std::max(max_nsb, s.nsb);
-    }
-    const uint32_t sb = split_sb(tiles, 1u, std::max(1u, cus));
+    for (const auto& s : g) tiles.push_back({((rows + 63u) / 64u) * ((s.n + 127u) / 128u), s.nsb});
+    const uint32_t sb = n128_split(tiles, cus);
     // 32-row tiles (small_gemm_tile_m): half a 64-row tile's weight operands at the least
     const double big = mmqh_time(g, rows, base.tile_m, 256u, base.sb,
                                  base.tile_m >= 128u ? kBig[t] : base.tile_m == 64u ? kMid[t] : 0.75 * kMid[t], cus);
@@ -1148,6 +1161,10 @@ int launch_quant(Ctx* c, const float* x, uint32_t ldx, const int32_t* src_rows, 
 // wave's registers)
 bool act_f16_wave(uint32_t rows, uint32_t k) { return k <= 4096u && rows >= 128u; }
 constexpr uint32_t kActWgThreads = 1024;  // of the row-per-workgroup kernels (quant.hpp)
+// The SiLU producers, a row per workgroup -> per wave (us): 4096 x 1024 30.5 ->
+// 14.9 (a quarter of the 1024 threads have values), 1024 x 1024 8.3 -> 6.2,
+// 2048 x 4096 24.7 -> 22.3; 1024 x 4096 17.7 per wave, 16.8 with 256 threads a row.
+bool silu_wave(uint32_t rows, uint32_t k) { return (k <= 2048u && rows >= 1024u) || (k <= 4096u && rows >= 2048u); }
 uint32_t act_f16_grid(uint32_t rows, bool wave) {
     return wave ? std::min<uint32_t>((rows + 3u) / 4u, 4096u) : std::min<uint32_t>(rows, 16384u);
 }
@@ -1224,8 +1241,10 @@ int launch_silu_act(Ctx* c, const float* gate, const float* up, uint32_t rows, u
            h ? reinterpret_cast<uint16_t*>(base + L.xsx) : nullptr,
            h ? reinterpret_cast<float*>(base + L.xrs) : nullptr,
            nullptr};
-    const uint32_t grid = h ? act_f16_grid(rows, false) : (quant_grid((uint64_t)rows * (k / 32u)) + 3u) / 4u;
-    return launch(c->silu_q, grid, 0, stream, &a, sizeof a, "rfxq_silu_and_mul_q8_1 launch", kActWgThreads);
+    const bool wave = h && silu_wave(rows, k);
+    const uint32_t grid = h ? act_f16_grid(rows, wave) : (quant_grid((uint64_t)rows * (k / 32u)) + 3u) / 4u;
+    return launch(wave ? c->silu_q_wave : c->silu_q, grid, 0, stream, &a, sizeof a, "rfxq_silu_and_mul_q8_1 launch",
+                  wave ? 256u : kActWgThreads);
 }
 
 // rfxq_moe_combine: out[t,:] = sum over the token's k pairs of w * pair_out row
@@ -1489,6 +1508,16 @@ uint32_t group_index(uint32_t ty, bool f16, uint32_t tile_m) {
     return (mix_f16(ty, tile_m) && f16 ? 0u : (uint32_t)type_index(ty)) + 3u * group_variant(f16, tile_m);
 }
 
+// median super-blocks per tile of a launch of (super-blocks per tile, tiles)
+uint32_t median_sb(std::vector<std::pair<uint32_t, uint32_t>> by_sb) {
+    uint64_t all = 0, acc = 0;
+    for (const auto& e : by_sb) all += e.second;
+    std::sort(by_sb.begin(), by_sb.end());
+    for (const auto& e : by_sb)
+        if ((acc += e.second) * 2u >= all) return e.first;
+    return by_sb.back().first;
+}
+
 // `ext` (optional, one per item): the items' x are caller activation buffers
 // (rfxq_act_q8_1_size layouts, already quantized): every GEMM takes an MMQ
 // kernel (f16 unless REFLEX_MMQ_F16=0) and the group quantizes nothing.
@@ -1570,7 +1599,7 @@ int build_gemm_group(const rfxq_gemm_item* items, uint32_t count, uint32_t rows,
     // than the launch's larger tiles (split as below)
     for (uint32_t t = 6u; t < kGroupFew && !o.quant_mma_splits && !general; t++) {
         std::vector<GemmShape> shapes;
-        std::vector<std::pair<uint32_t, uint32_t>> tn;
+        std::vector<std::pair<uint32_t, uint32_t>> tn, by_sb;
         uint32_t ty = 0, tiles = 0, max_nsb = 0;
         for (uint32_t i = 0; i < count; i++) {
             if (item_act[i] == ~0u || item_kernel[i] != t) continue;
@@ -1579,10 +1608,12 @@ int build_gemm_group(const rfxq_gemm_item* items, uint32_t count, uint32_t rows,
             const uint32_t bm = group_tile_m(t);
             tn.push_back({((rows + bm - 1u) / bm) * ((shapes.back().n + 255u) / 256u), shapes.back().nsb});
             tiles += tn.back().first;
+            by_sb.push_back({shapes.back().nsb, tn.back().first});
             max_nsb = std::max(max_nsb, shapes.back().nsb);
         }
         if (shapes.empty()) continue;
-        const uint32_t sb = 2u * tiles < cus ? split_sb(tn, 2u, 2u * std::max(cus, 1u)) : max_nsb;
+        const uint32_t med = median_sb(by_sb);  // (the larger tiles split rows over 3x it, below)
+        const uint32_t sb = 2u * tiles < cus ? split_sb(tn, 2u, 2u * std::max(cus, 1u)) : max_nsb > 3u * med ? med : max_nsb;
         if (n128_sb(shapes, ty, rows, cus, {group_tile_m(t), sb}))
             for (uint32_t i = 0; i < count; i++)
                 if (item_act[i] != ~0u && item_kernel[i] == t) item_kernel[i] = kGroupN128 + (uint32_t)type_index(ty);
@@ -1633,7 +1664,7 @@ int build_gemm_group(const rfxq_gemm_item* items, uint32_t count, uint32_t rows,
         // one split size for the launch, so its workgroups take alike
         std::vector<std::pair<uint32_t, uint32_t>> tn;
         for (const auto& d : v) tn.push_back({d.tiles_m * d.tiles_n, d.k / 256u});
-        uint32_t w_sb = t >= kGroupN128 ? split_sb(tn, 1u, std::max(cus, 1u))
+        uint32_t w_sb = t >= kGroupN128 ? n128_split(tn, cus)
                                         : split_sb(tn, group_tile_m(t) == 32u ? 1u : 2u, 2u * std::max(cus, 1u));
         if (t == kGroupFew) w_sb = std::min(w_sb, few_max_sb(rows));
         uint32_t wg = 0;
@@ -1662,19 +1693,8 @@ int build_gemm_group(const rfxq_gemm_item* items, uint32_t count, uint32_t rows,
         auto& v = g->descs[t];
         if (v.size() < 2u || split_small[t]) continue;
         std::vector<std::pair<uint32_t, uint32_t>> by_sb;  // (super-blocks per tile, tiles)
-        uint64_t all = 0;
-        for (const auto& d : v) {
-            by_sb.push_back({d.sb_per_split, d.tiles_m * d.tiles_n * d.splits});
-            all += by_sb.back().second;
-        }
-        std::sort(by_sb.begin(), by_sb.end());
-        uint64_t acc = 0;
-        uint32_t med = by_sb.back().first;
-        for (const auto& e : by_sb)
-            if ((acc += e.second) * 2u >= all) {
-                med = e.first;
-                break;
-            }
+        for (const auto& d : v) by_sb.push_back({d.sb_per_split, d.tiles_m * d.tiles_n * d.splits});
+        const uint32_t med = median_sb(by_sb);
         bool changed = false;
         for (uint32_t i = 0; i < v.size(); i++) {
             MmqDesc& d = v[i];
@@ -2300,8 +2320,9 @@ int rfxq_silu_and_mul_q8_1(const float* gate, const float* up, uint32_t rows, ui
     } a = {gate, up, rows, k, reinterpret_cast<int8_t*>(b + L.xq), reinterpret_cast<uint32_t*>(b + L.xds),
            reinterpret_cast<uint16_t*>(b + L.xh), reinterpret_cast<uint16_t*>(b + L.xsx),
            reinterpret_cast<float*>(b + L.xrs), y};
-    if (int rc = launch(c->silu_q, act_f16_grid(rows, false), 0, stream, &a, sizeof a, "rfxq_silu_and_mul_q8_1 launch",
-                        kActWgThreads))
+    const bool wave = silu_wave(rows, k);
+    if (int rc = launch(wave ? c->silu_q_wave : c->silu_q, act_f16_grid(rows, wave), 0, stream, &a, sizeof a,
+                        "rfxq_silu_and_mul_q8_1 launch", wave ? 256u : kActWgThreads))
         return rc;
     return ok();
 }

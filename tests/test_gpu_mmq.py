@@ -345,6 +345,41 @@ def test_gemm_few_rows_many_tiles(rq, ty, m, n, k):
     assert float((y - ref).abs().max()) <= 1e-5 * float(ref.abs().max())
 
 
+@pytest.mark.parametrize("rows,k", [(1024, 256), (1023, 2048), (1025, 2304), (2049, 4096), (3, 16640), (1024, 768)])
+def test_activation_producers_wave_and_workgroup(rq, rows, k):
+    """The producers' layouts do not depend on how many rows a launch has (a row per wave or per workgroup,
+    registers or two reads): the first and last row equal those of a one-row call, byte for byte."""
+    g, u = _dev(synth.activations(rows * k, 980)), _dev(synth.activations(rows * k, 981))
+
+    def parts(act, r):
+        a16 = lambda v: (v + 255) // 256 * 256
+        out, o = [], 0
+        for per in (k, k // 32 * 4, 2 * k, k // 256 * 32, 4):  # int8, d | s, f16, block sums, row scale
+            out.append([act[o + i * per:o + (i + 1) * per].cpu() for i in (0, r - 1)])
+            o += a16(r * per)
+        return out
+
+    for make in (lambda r: rq.quantize_act_q8_1(g[r], g[r].numel() // k, k),
+                 lambda r: rq.silu_and_mul_q8_1(g[r], u[r], g[r].numel() // k, k)[0]):
+        full = parts(make(slice(None)), rows)
+        first, last = parts(make(slice(0, k)), 1), parts(make(slice((rows - 1) * k, rows * k)), 1)
+        for f, a, b in zip(full, first, last):
+            assert torch.equal(f[0], a[0]) and torch.equal(f[1], b[0])
+
+
+def test_group_of_short_and_long_rows(rq, orc):
+    """A Q8_0 group of K = 256, 1280 and 4864 on 64 x 128 tiles: ranges follow the shortest row."""
+    m, items, refs = 40, [], []
+    for i, (n, k) in enumerate(((640, 1280), (130, 256), (384, 4864))):
+        w_np = synth.weights(Q8_0, n, k, 990 + i)
+        x_np = synth.activations(m * k, 995 + i).reshape(m, k)
+        items.append((_dev(x_np.reshape(-1)), _weight(rq, Q8_0, w_np, n, k), torch.empty(m * n, device=DEV)))
+        refs.append(orc.reference_gemm(Q8_0, w_np, n, k, x_np))
+    rq.gemm_batch(items, m)
+    for (_, w, y), ref in zip(items, refs):
+        assert orc.rel_err_row_l2(y.cpu().numpy().reshape(m, -1), ref) < TOL
+
+
 @pytest.mark.parametrize("ty", [Q4K, Q6K, Q8_0])
 def test_gemm_few_rows_workspaces(rq, ty):
     """Workspaces that hold the 32-row tiles' plan: the advertised bytes with an output over its input; none for
