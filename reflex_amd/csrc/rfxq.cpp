@@ -872,7 +872,8 @@ uint32_t tile_bn(bool f16) { return f16 ? 256u : 128u; }
 // - otherwise the f16-activation kernels (PATH_MMQ_F16: Q4_K, Q6_K and Q8_0,
 //   the default): 32-row tiles up to 32 rows (the fused
 //   few-row form: each weight read once for all rows), 64-row tiles up to
-//   64, 128-row tiles above,
+//   64, 128-row tiles above; plan_gemm and build_gemm_group run them on the
+//   few-row kernel (few_wins) or 64 x 128 tiles (n128_sb) where those are faster,
 //   or the int8 kernels (PATH_MMQ_INT8; 64-row tiles with
 //   REFLEX_QUANT_MMA_TILE=64);
 // - split-K: none once the tiles cover half the CUs (each CU holds two
@@ -2419,7 +2420,6 @@ int rfxq_gemm_gate_up_silu_q8_1(const void* act, uint32_t rows, const rfxq_weigh
         return rfxq_quantize_act_q8_1(y, rows, ffn, act_out, stream);
     }
     // separate GEMMs into the workspace, then SiLU·up into y and act_out
-    // (not in place: rfxq_silu_and_mul_q8_1 reads its inputs once per layout)
     const uint64_t u_bytes = align256((uint64_t)rows * ffn * 4u);
     const uint64_t need = rfxq_gemm_gate_up_silu_workspace_size(gate, rows);
     void* ws = workspace;
