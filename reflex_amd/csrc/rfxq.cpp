@@ -917,24 +917,71 @@ uint32_t few_max_sb(uint32_t rows) { return rows > 32u ? 0u : rows > 16u ? 4u : 
 uint32_t few_lds(uint32_t rows, uint32_t sb) {
     return 128u + std::max(16384u, rows * (sb * 544u + 16u));  // (results pass through 4 KB per wave)
 }
-// Whether one launch of `tiles` 32 x 256 tiles (`load` super-blocks over all
-// of them, the longest row max_nsb) runs on the few-row kernel. It keeps more
-// weight bytes in flight than the 32-row tiles, but each of its workgroups
-// brings the f32 rows in itself, and its short ranges write more partials:
-// both grow with the rows, and the tiles catch up once they fill the CUs.
+// Whether one launch of 32 x 256 tiles runs on the few-row kernel. It keeps more weight bytes in flight than the 32-row tiles,
+// but each of its workgroups brings the f32 rows in itself, and its short
+// ranges write more partials: both grow with the rows.
+// - Tiles for less than half the CUs: the tiles split K as well, and the
+//   few-row kernel is faster but for many rows of long launches (an 8B layer,
+//   3300 super-blocks: 24 rows 78 -> 74 us, 32 rows 78 -> 79).
+// - Up to a tile per CU: the tiles run unsplit, so their time is a whole row's
+//   whatever their number, and the few-row kernel's is its longest range (two
+//   workgroups a CU), its partials and its results. The constants (us: fixed,
+//   per super-block of a row, per super-block of a range, per row and range of
+//   a CU, per row and tile of a CU) are fitted to 4100 launches of 129 to 256
+//   tiles (1 to 56 super-blocks, 5 to 32 rows). Of those and 2050 launches of
+//   fewer tiles 34 are over 3% slower for the choice, 8% at the most. Launches
+//   of one range a row write no partials and always win. At exactly half the CUs
+//   (the fewest tiles that run unsplit) they are slowest, hence its own line.
+// - More tiles fill every CU.
 // Measured, 32-row tiles -> few-row kernel (us), Q4_K / Q6_K / Q8_0:
 //   4096 x 4096       16 rows 15 -> 12 / 18 -> 16 / 17 -> 15;   32: 17 -> 15 / 19 -> 18 / 19 -> 18
-//   32768 x 2048      16 rows 25 -> 20 / 37 -> 26 / 44 -> 31;   32: 26 -> 25 / 37 -> 30 / 45 -> 34
-//   8B layer (3300 super-blocks of tiles)  24 rows 78 -> 74, Q8_0 90 -> 88;  32: 78 -> 79, 91 -> 93
-//   65536 x 1024      16 rows 18 -> 23 / 26 -> 28 / 26 -> 32;   32: 19 -> 30 / 26 -> 35 / 26 -> 37
-//   65536 x 2048       8 rows 29 -> 26 / 41 -> 38 / 46 -> 43;   16: 29 -> 31 / 41 -> 41 / 46 -> 46
-//   65536 x 4096      16 rows 50 -> 47 / 75 -> 71 / 104 -> 92;  32: 48 -> 61 / 76 -> 82 / 106 -> 107
+//   32768 x 2048      16 rows 29 -> 23 / 45 -> 28 / 55 -> 38;   32: 30 -> 27 / 45 -> 34 / 56 -> 43
+//   40960 x 1024       8 rows 18 -> 19 / 27 -> 24 / 32 -> 32;   32: 19 -> 28 / 28 -> 33 / 34 -> 40
+//   49152 x 2048      16 rows 31 -> 31 / 46 -> 42 / 54 -> 52;   32: 31 -> 39 / 47 -> 49 / 55 -> 59
+//   49152 x 4096      16 rows 50 -> 46 / 85 -> 73 / 106 -> 96;  32: 52 -> 57 / 86 -> 74 / 107 -> 93
+//   65280 x 1024       8 rows 20 -> 21 / 29 -> 28 / 34 -> 34;   32: 20 -> 31 / 30 -> 38 / 35 -> 45
+//   65280 x 4096      16 rows 55 -> 50 / 89 -> 76 / 109 -> 100; 32: 56 -> 73 / 91 -> 94 / 110 -> 116
 //   128256 x 4096      8 rows 86 -> 79 / 167 -> 131 / 208 -> 180;   16: 85 -> 88 / 169 -> 140 / 209 -> 188
 //   151936 x 1024     16 rows 34 -> 33 / 62 -> 49 / 64 -> 53;   32: 35 -> 40 / 64 -> 54 / 66 -> 59
-bool few_wins(uint32_t tiles, uint64_t load, uint32_t max_nsb, uint32_t rows, bool q4k, uint32_t cus) {
-    if (tiles < cus) return rows <= 24u || load <= 8ull * cus;
-    if (rows <= (q4k ? 8u : 16u)) return max_nsb > 4u || tiles >= 2u * cus;
-    return !q4k && max_nsb <= 4u && tiles >= 2u * cus;  // (one range: no partials)
+struct FewShape {
+    uint32_t tiles, nsb;  // of 256 columns, super-blocks per row
+    int type;             // type_index
+};
+bool few_wins(const std::vector<FewShape>& gemms, uint32_t rows, uint32_t cus) {
+    uint32_t tiles = 0, max_nsb = 0;
+    uint64_t load = 0;
+    bool q4k = false;
+    std::vector<std::pair<uint32_t, uint32_t>> tn;
+    for (const auto& g : gemms) {
+        tiles += g.tiles;
+        load += (uint64_t)g.tiles * g.nsb;
+        max_nsb = std::max(max_nsb, g.nsb);
+        q4k |= g.type == 0;
+        tn.push_back({g.tiles, g.nsb});
+    }
+    if (tiles > cus) {
+        if (rows <= (q4k ? 8u : 16u)) return max_nsb > 4u || tiles >= 2u * cus;
+        return !q4k && max_nsb <= 4u && tiles >= 2u * cus;  // (one range: no partials)
+    }
+    if (rows > 24u && load > 8ull * cus) return false;
+    if (2u * tiles < cus) return true;
+    static const double kCost[3][5] = {{2.4, 2.1, 2.4, 0.15, 0.15}, {2.6, 3.5, 4.0, 0.089, 0.22}, {4.0, 4.3, 5.3, 0.033, 0.33}};
+    const uint32_t sb = std::min(split_sb(tn, 1u, 2u * std::max(cus, 1u)), few_max_sb(rows));
+    uint64_t ranges = 0;
+    double row_max = 0.0, row_sum = 0.0, range_max = 0.0;
+    for (const auto& g : gemms) {
+        const uint32_t s = (g.nsb + sb - 1u) / sb;
+        ranges += (uint64_t)g.tiles * s;
+        row_max = std::max(row_max, kCost[g.type][1] * g.nsb);
+        row_sum += kCost[g.type][1] * g.nsb * g.tiles;
+        range_max = std::max(range_max, kCost[g.type][2] * ((g.nsb + s - 1u) / s));
+    }
+    if (ranges == tiles) return true;
+    if (2u * tiles == cus) return q4k ? rows <= 12u || load >= 8ull * tiles : rows <= 20u || load >= 4ull * tiles;
+    const double* c = kCost[q4k ? 0 : gemms[0].type];
+    const double rounds = (double)((ranges + 2u * cus - 1u) / (2u * cus));
+    // (a group's tiles end between its longest row and the mean one)
+    return c[0] - 0.5 * (row_max + row_sum / tiles) + range_max * rounds + (c[3] * ranges + c[4] * tiles) * rows / cus < 0.0;
 }
 
 // Row tile of one grouped MoE GEMM, `pairs` routed rows over `experts`
@@ -1349,7 +1396,7 @@ GemmPlan plan_gemm(const Ctx* c, const rfxq_weight* w, uint32_t rows, const rfxq
     if (p.f16 && !general && !in_place && few_max_sb(rows)) {
         const uint32_t tiles = (n + 255u) / 256u;
         if (forced) p.few = p.pol.sb_per_split <= few_max_sb(rows);
-        else if (few_wins(tiles, (uint64_t)tiles * nsb, nsb, rows, w->ggml_type == RFXQ_TYPE_Q4_K, cus)) {
+        else if (few_wins({{tiles, nsb, type_index(w->ggml_type)}}, rows, cus)) {
             p.few = true;
             sb = std::min(split_sb({{tiles, nsb}}, 1u, 2u * std::max(cus, 1u)), few_max_sb(rows));
         }
@@ -1579,18 +1626,12 @@ int build_gemm_group(const rfxq_gemm_item* items, uint32_t count, uint32_t rows,
         if (!f16) g->acts[ai].need_i8 = true;
     }
     // the few-row kernel, or tiles, for all its GEMMs (few_wins)
-    uint32_t few_tiles = 0, few_nsb = 0;
-    uint64_t few_load = 0;
-    bool few_q4k = false;
-    for (uint32_t i = 0; i < count; i++) {
-        if (item_act[i] == ~0u || item_kernel[i] != kGroupFew) continue;
-        const uint32_t tiles = (items[i].w->out_features + 255u) / 256u, nsb = items[i].w->in_features / 256u;
-        few_tiles += tiles;
-        few_load += (uint64_t)tiles * nsb;
-        few_nsb = std::max(few_nsb, nsb);
-        few_q4k |= items[i].w->ggml_type == RFXQ_TYPE_Q4_K;
-    }
-    const bool few_kept = o.quant_mma_splits || few_wins(few_tiles, few_load, few_nsb, rows, few_q4k, cus);
+    std::vector<FewShape> few_gemms;
+    for (uint32_t i = 0; i < count; i++)
+        if (item_act[i] != ~0u && item_kernel[i] == kGroupFew)
+            few_gemms.push_back({(items[i].w->out_features + 255u) / 256u, items[i].w->in_features / 256u,
+                                 type_index(items[i].w->ggml_type)});
+    const bool few_kept = o.quant_mma_splits || (!few_gemms.empty() && few_wins(few_gemms, rows, cus));
     for (uint32_t i = 0; i < count; i++) {
         if (item_act[i] == ~0u) continue;
         if (item_kernel[i] == kGroupFew && !few_kept) item_kernel[i] = group_index(items[i].w->ggml_type, true, 32u);

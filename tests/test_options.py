@@ -200,6 +200,23 @@ def test_workspace_of_few_rows_fits_the_scratch(rq, ty, n, k, rows):
     assert 0 < rq.gemm_workspace_size(w, rows) <= 128 << 20
 
 
+@pytest.mark.parametrize("ty,n,k,rows,few", [
+    # measured, 32-row tiles -> few-row kernel (us): 20 -> 25, 20 -> 31, 19 -> 25, 56 -> 65, 31 -> 41, 30 -> 37, 35 -> 42
+    (Q4K, 65280, 1024, 16, False), (Q4K, 65280, 1024, 32, False), (Q4K, 49152, 1024, 24, False),
+    (Q4K, 65280, 4096, 24, False), (Q4K, 57344, 2048, 32, False), (Q6K, 61440, 1024, 32, False),
+    (Q8_0, 65280, 1024, 24, False),
+    # 30 -> 27, 55 -> 44, 18 -> 15, 89 -> 76, 46 -> 40, 33 -> 28, 104 -> 72
+    (Q4K, 32768, 2048, 32, True), (Q4K, 65280, 4096, 8, True), (Q4K, 16384, 2048, 5, True),
+    (Q6K, 65280, 4096, 16, True), (Q6K, 40960, 2048, 32, True), (Q8_0, 32768, 1024, 32, True),
+    (Q8_0, 40960, 4096, 8, True)])
+def test_few_row_kernel_is_used_where_it_is_faster(rq, ty, n, k, rows, few):
+    """Up to a 256-column tile per CU: the few-row kernel's ranges need workspace for their partials, the unsplit
+    tiles for the f16 layout of the rows only (a 16384 x 2048 matrix splits K either way)."""
+    import torch
+    w = rq.Weight(rq.GgmlType(ty), torch.empty(16, dtype=torch.uint8), [k, n])
+    assert (rq.gemm_workspace_size(w, rows) >= 2 * rows * n * 4) == few
+
+
 def test_policy_errors(rq):
     with pytest.raises(rq.GgmlError):
         rq.gemm_policy(2, 1024, 1024, 512)
