@@ -1189,7 +1189,7 @@ RFXQ_MMQH_MIX_ENTRY(rfxq_mmqh_mix_m32, 1, 3)
 
 // 64 x 128 tiles (32 columns a wave), any type: for GEMMs whose larger tiles
 // would be so few that K is cut into many ranges, whose partial sums then go
-// through memory (the host's choice, n128_better). A tile runs at two thirds
+// through memory (the host's choice, n128_sb). A tile runs at two thirds
 // of the 128 x 256 tile's rate per CU (its weight operands serve 64 rows, its
 // activation reads 32 columns a wave), but there are four times as many: 512
 // rows of an 8B o_proj (4096 x 4096) take 28.6 us as 256 tiles, without a

@@ -1025,36 +1025,74 @@ uint32_t small_gemm_tile_m(uint32_t tile_m, uint32_t rows, uint32_t n, uint32_t 
 
 // ---- 64 x 128 tiles instead of the larger ones
 //
-// Estimated time (us) of one f16 launch of GEMMs {n, super-blocks per row} of
-// `rows` rows on `bm` x `bn` tiles with ranges of `sb` super-blocks. A CU
-// takes `c` us per tile and super-block, whether its workgroups run side by
-// side or in turn; a launch of more workgroups than CUs ends later than its
-// average CU (fitted: 0.85 of the average load and 0.35 of a workgroup).
-// Partial sums of split GEMMs are written and read once at 5 TB/s.
+// Estimated time (us, less what all tiles take alike) of one f16 launch of
+// GEMMs {n, super-blocks per row} of `rows` rows on `bm` x `bn` tiles with
+// ranges of `sb` super-blocks and the tiles' constants c. The launch ends with
+// its slowest XCD (each takes an eighth of the tiles, contiguous ones), whose
+// workgroups come to its CUs in rounds of one per CU: a launch of a few more
+// than a round ends a whole workgroup later (14336 x 4096 Q8_0 at 400 rows: 784
+// tiles of 64 x 128, four rounds, 169 us; 106 us as 224 of 128 x 256). A longer
+// workgroup than the XCD's mean ends late by as much more as there are fewer
+// rounds. Partial sums of split GEMMs are written and read once.
 struct GemmShape {
     uint32_t n, nsb;
 };
-double mmqh_time(const std::vector<GemmShape>& g, uint32_t rows, uint32_t bm, uint32_t bn, uint32_t sb, double c,
-                 uint32_t cus) {
+struct MmqhCost {
+    // us: fixed, per MB of partials, per super-block of an XCD's rounds, of its CUs' load, of the mean workgroup
+    double fixed, part, round, load, mean;
+};
+double mmqh_time(const std::vector<GemmShape>& g, uint32_t rows, uint32_t bm, uint32_t bn, uint32_t sb,
+                 const MmqhCost& c, uint32_t cus) {
+    struct Run {
+        uint64_t wgs;
+        double mean;  // super-blocks
+        uint32_t longest;
+    };
+    std::vector<Run> runs;
     uint64_t wgs = 0;
-    double load = 0.0, part = 0.0;
-    uint32_t longest = 0;
+    double total = 0.0, part = 0.0;
     for (const auto& s : g) {
         const uint64_t tiles = (uint64_t)((rows + bm - 1u) / bm) * ((s.n + bn - 1u) / bn);
         const uint32_t splits = (s.nsb + sb - 1u) / sb;
+        runs.push_back({tiles * splits, (double)s.nsb / splits, (s.nsb + splits - 1u) / splits});
         wgs += tiles * splits;
-        load += (double)tiles * s.nsb;
-        longest = std::max(longest, std::min(sb, s.nsb));
-        if (splits > 1u) part += 8.0 * splits * rows * s.n / 5e6;
+        total += (double)tiles * s.nsb;
+        if (splits > 1u) part += 8e-6 * splits * rows * s.n;
     }
-    return 3.0 + part + c * (wgs <= cus ? longest : 0.85 * load / cus + 0.35 * longest);
+    const uint64_t xcd_cus = std::max(1u, cus / 8u);
+    double rounds = 0.0, load = 0.0;
+    size_t at = 0;
+    for (uint32_t x = 0; x < 8u; x++) {
+        const uint64_t n = wgs / 8u + (x < wgs % 8u ? 1u : 0u);
+        double sum = 0.0;
+        uint32_t longest = 0;
+        for (uint64_t left = n; left != 0u;) {
+            if (runs[at].wgs == 0u) {
+                at++;
+                continue;
+            }
+            const uint64_t take = std::min(left, runs[at].wgs);
+            sum += (double)take * runs[at].mean;
+            longest = std::max(longest, runs[at].longest);
+            runs[at].wgs -= take;
+            left -= take;
+        }
+        if (n == 0u) continue;
+        const double r = (double)((n + xcd_cus - 1u) / xcd_cus), mean = sum / n;
+        rounds = std::max(rounds, r * mean + (longest - mean) / r);
+        load = std::max(load, sum / xcd_cus);
+    }
+    return c.fixed + c.part * part + c.round * rounds + c.load * load + c.mean * total / wgs;
 }
 
 // Super-blocks per range on 64 x 128 tiles for the GEMMs of one type and one
-// launch, or 0 where the larger tiles `base` {rows, super-blocks per range}
-// are estimated faster. 64 x 128 tiles split K only as far as there are idle
-// CUs. us per tile and super-block, measured (Q4_K / Q6_K / Q8_0): 128 x 256
-// 4.1 / 5.5 / 7.5, 64 x 256 2.9 / 4.0 / 4.5, 64 x 128 1.65 / 2.35 / 2.5; main
+// launch, or 0 where they are not estimated 4% (10%: 32-row tiles) faster than the larger tiles
+// `base` {rows, super-blocks per range}. 64 x 128 tiles split K only as far as
+// there are idle CUs. The constants are fitted to the measured differences of
+// 2550 single GEMMs (n 64-14336, K 256-14336, 33-1500 rows) and 2604 groups
+// (parts of a layer to eight layers, 33-1024 rows): the choices run 1.25x and
+// 1.13x faster than the larger tiles on average, 0.3% behind the faster of the
+// two; 52 are over 3% slower, 12% at the most but for two groups (20-24%). Main
 // launch and reduce at 4096 x 4096 Q4_K: 64 rows 11.5 + 3.5 -> 8.1 + 3.5 us,
 // 128 rows 15.2 + 4.5 -> 10.9 + 3.5, 512 rows 30.6 + 15.5 -> 28.6 + 0, 1024
 // rows 42.9 + 10 -> 50.2 + 0; 4096 x 14336 Q6_K at 512 rows stays on 128 x 256
@@ -1078,16 +1116,19 @@ uint32_t n128_split(const std::vector<std::pair<uint32_t, uint32_t>>& tiles_nsb,
     return wgs <= cus && 4u * sb <= 5u * shortest ? sb : std::min(sb, shortest);
 }
 uint32_t n128_sb(const std::vector<GemmShape>& g, uint32_t ty, uint32_t rows, uint32_t cus, TileSplit base) {
-    static const double kBig[3] = {4.1, 5.5, 7.5}, kMid[3] = {2.9, 4.0, 4.5}, kSmall[3] = {1.65, 2.35, 2.5};
+    // [type][128 x 256, 64 x 256, 32 x 256, 64 x 128]
+    static const MmqhCost kCost[3][4] = {
+        {{2.2, 0.23, 2.36, 0.88, 0.57}, {0.27, 0.27, 1.8, 0.53, 0.67}, {0.39, 0.2, 0.93, 0.73, 0.37}, {0, 0.27, 0.68, 0.54, 0.49}},
+        {{2.57, 0.22, 4.3, 0.058, 0.61}, {1.2, 0.3, 3.6, 0.36, 0}, {-1.33, 0.36, 3.03, 0, 1.07}, {0, 0.31, 1.66, 0.43, 0.04}},
+        {{3.58, 0.23, 4.01, 0, 0.82}, {0.82, 0.32, 4.09, 0.19, 0}, {-0.33, 0.3, 2.23, 0, 1.71}, {0, 0.29, 1.77, 0.043, 0.39}}};
     if (rows <= 32u) return 0u;
     const int t = type_index(ty);
     std::vector<std::pair<uint32_t, uint32_t>> tiles;
     for (const auto& s : g) tiles.push_back({((rows + 63u) / 64u) * ((s.n + 127u) / 128u), s.nsb});
     const uint32_t sb = n128_split(tiles, cus);
-    // 32-row tiles (small_gemm_tile_m): half a 64-row tile's weight operands at the least
-    const double big = mmqh_time(g, rows, base.tile_m, 256u, base.sb,
-                                 base.tile_m >= 128u ? kBig[t] : base.tile_m == 64u ? kMid[t] : 0.75 * kMid[t], cus);
-    return mmqh_time(g, rows, 64u, 128u, sb, kSmall[t], cus) < big ? sb : 0u;
+    const int b = base.tile_m >= 128u ? 0 : base.tile_m == 64u ? 1 : 2;
+    const double big = mmqh_time(g, rows, base.tile_m, 256u, base.sb, kCost[t][b], cus);
+    return mmqh_time(g, rows, 64u, 128u, sb, kCost[t][3], cus) < (b == 2 ? 0.9 : 0.96) * big ? sb : 0u;
 }
 
 // raw bytes of a weight matrix

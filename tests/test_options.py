@@ -217,6 +217,23 @@ def test_few_row_kernel_is_used_where_it_is_faster(rq, ty, n, k, rows, few):
     assert (rq.gemm_workspace_size(w, rows) >= 2 * rows * n * 4) == few
 
 
+@pytest.mark.parametrize("ty,n,k,rows,n128", [
+    # measured, larger tiles -> 64 x 128 (us): 193 -> 306, 75 -> 92, 79 -> 92, 75 -> 93, 82 -> 94
+    (Q8_0, 14336, 14336, 160, False), (Q8_0, 14336, 4096, 160, False), (Q8_0, 8430, 4096, 300, False),
+    (Q8_0, 4096, 4096, 705, False), (Q8_0, 4096, 14336, 200, False),
+    # 48 -> 39, 40 -> 29, 43 -> 31, 118 -> 106, 50 -> 36
+    (Q4K, 8430, 4096, 128, True), (Q6K, 8430, 4096, 33, True), (Q8_0, 8430, 4096, 33, True),
+    (Q8_0, 14336, 14336, 48, True), (Q4K, 4096, 4096, 512, True)])
+def test_64x128_tiles_are_used_where_they_are_faster(rq, ty, n, k, rows, n128):
+    """GEMMs whose larger tiles split K: their plan's workspace holds the policy's partial sums, the 64 x 128 tiles'
+    fewer."""
+    import torch
+    w = rq.Weight(rq.GgmlType(ty), torch.empty(16, dtype=torch.uint8), [k, n])
+    p = rq.gemm_policy(ty, k, n, rows)
+    assert p["splits"] > 1
+    assert (rq.gemm_workspace_size(w, rows) < p["splits"] * rows * n * 4) == n128
+
+
 def test_policy_errors(rq):
     with pytest.raises(rq.GgmlError):
         rq.gemm_policy(2, 1024, 1024, 512)
