@@ -123,6 +123,11 @@ typedef struct rfxq_gemm_policy {
 int rfxq_gemm_policy_for(uint32_t ggml_type, uint32_t in_features, uint32_t out_features, uint32_t rows,
                          uint32_t compute_units, rfxq_gemm_policy* out);
 
+/* Test hook: the tiles and splits rfxq_gemm runs on the current device (256
+ * compute units before rfxq_init) for an output apart from the input and a
+ * workspace of the reported size. */
+int rfxq_gemm_plan_policy(const rfxq_weight* w, uint32_t rows, rfxq_gemm_policy* out);
+
 /* (elements per block, bytes per block) of a ggml type (src/gguf.rs:366-400). */
 int rfxq_block_dims(uint32_t ggml_type, uint32_t* block_elems, uint32_t* block_bytes);
 
@@ -176,8 +181,8 @@ void rfxq_gemv_plan_destroy(rfxq_gemv_plan* plan);
  * = d_bits | s_bits << 16 (d = amax/127, q = roundf(x/d), s = d*sum(q)). */
 int rfxq_quantize_q8_1(const float* x, uint32_t rows, uint32_t k, int8_t* xq, uint32_t* xds, hipStream_t stream);
 
-/* Bytes of workspace rfxq_gemm needs for this weight and row count (an output
- * over the input included). */
+/* Bytes of workspace rfxq_gemm needs for this weight and row count, on the
+ * policy's plan and on the one it runs (rfxq_gemm_plan_policy). */
 uint64_t rfxq_gemm_workspace_size(const rfxq_weight* w, uint32_t rows);
 
 /* Model::gemm (src/model/kernels.rs:2197) on a quantized-resident weight:
@@ -198,8 +203,8 @@ int rfxq_gemm(const float* x, uint64_t x_len, const rfxq_weight* w, uint32_t row
  * hipMalloc). It has no counterpart in the reference. Same path, kernels and
  * results as rfxq_gemm with a NULL workspace; the workspace is a fixed
  * 128 MiB device array per GPU (a file-scope __device__ array, held until the
- * process ends), so GEMMs whose workspace (rfxq_gemm_workspace_size) exceeds
- * it fail with RFXQ_ERR_INVALID_INPUT. The device must be initialised first
+ * process ends), so GEMMs that need more than it holds on every plan fail
+ * with RFXQ_ERR_INVALID_INPUT. The device must be initialised first
  * (rfxq_init), which resolves the array's address. Every call on a GPU shares
  * its array and leaves its contents there: calls that overlap on one GPU (on
  * different streams) race. */

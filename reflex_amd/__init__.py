@@ -63,6 +63,7 @@ SIGNATURES = {
     "rfxq_get_options": (_I, [ctypes.POINTER(RfxqOptions)]),
     "rfxq_set_options": (_I, [ctypes.POINTER(RfxqOptions)]),
     "rfxq_gemm_policy_for": (_I, [_U32, _U32, _U32, _U32, _U32, ctypes.POINTER(RfxqGemmPolicy)]),
+    "rfxq_gemm_plan_policy": (_I, [_WP, _U32, ctypes.POINTER(RfxqGemmPolicy)]),
     "rfxq_block_dims": (_I, [_U32, ctypes.POINTER(_U32), ctypes.POINTER(_U32)]),
     "rfxq_dequantize": (_I, [_U32, _P, _U64, _P, _I, _P]),
     "rfxq_gemv_to": (_I, [_P, _U64, _WP, _P, _P]),

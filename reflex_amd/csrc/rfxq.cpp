@@ -2209,18 +2209,34 @@ int rfxq_quantize_q8_1(const float* x, uint32_t rows, uint32_t k, int8_t* xq, ui
     return ok();
 }
 
+// the current device's context, or NULL where it is not initialised
+static Ctx* loaded_ctx() {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+    std::lock_guard<std::mutex> lk(g_mu);
+    auto it = g_ctx.find(dev);
+    return it != g_ctx.end() ? it->second.get() : nullptr;
+}
+
+int rfxq_gemm_plan_policy(const rfxq_weight* w, uint32_t rows, rfxq_gemm_policy* out) {
+    if (!w || !out) return fail(RFXQ_ERR_INVALID_INPUT, "gemm_plan_policy: NULL weight or output");
+    rfxq_gemm_policy general;  // checks the type and the sizes
+    if (int rc = rfxq_gemm_policy_for(w->ggml_type, w->in_features, w->out_features, rows, 256u, &general)) return rc;
+    rfxq_options o;
+    if (int rc = get_options(&o)) return rc;
+    *out = plan_gemm(loaded_ctx(), w, rows, o).pol;
+    return ok();
+}
+
 uint64_t rfxq_gemm_workspace_size(const rfxq_weight* w, uint32_t rows) {
     if (!w || rows == 0) return 0;
-    Ctx* c = nullptr;
-    int dev = 0;
-    if (hipGetDevice(&dev) == hipSuccess) {
-        std::lock_guard<std::mutex> lk(g_mu);
-        auto it = g_ctx.find(dev);
-        if (it != g_ctx.end()) c = it->second.get();
-    }
+    const Ctx* c = loaded_ctx();
     if (!options_ok()) return 0;
-    // with an output over its input too (both layouts are never held at once)
-    const GemmPlan p = plan_gemm(c, w, rows, opt()), q = plan_gemm(c, w, rows, opt(), true);
+    // the policy's own plan too: it runs an output over its input, and a buffer
+    // sized for the most rows a caller will have then holds fewer rows' longer
+    // splits (4096 x 4096 Q4_K: 64 x 128 tiles need 4 MB at 512 rows, which do
+    // not split, and 9 MB at 64, which do; the policy 71 and 17 MB)
+    const GemmPlan p = plan_gemm(c, w, rows, opt()), q = plan_gemm(c, w, rows, opt(), true, true);
     return p.pol.path == PATH_GEMV_ROWS ? 0 : std::max(p.total, q.total);
 }
 

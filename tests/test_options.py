@@ -3,6 +3,7 @@ environment is parsed once, strictly, with the reference's messages
 (QuantMmaKernels::from_env, src/model/kernels.rs:747-802;
 quant_fused_max_rows, :4186-4194), and rfxq_gemm_policy_for makes the
 documented choices. No compute call runs here."""
+import ctypes
 import os
 import subprocess
 import sys
@@ -200,6 +201,18 @@ def test_workspace_of_few_rows_fits_the_scratch(rq, ty, n, k, rows):
     assert 0 < rq.gemm_workspace_size(w, rows) <= 128 << 20
 
 
+def _shape(rq, ty, n, k):
+    import torch
+    return rq.Weight(rq.GgmlType(ty), torch.empty(16, dtype=torch.uint8), [k, n])
+
+
+def _plan_policy(rq, w, rows):
+    from reflex_amd import RfxqGemmPolicy
+    p = RfxqGemmPolicy()
+    assert rq.lib().rfxq_gemm_plan_policy(w.cref(), rows, ctypes.byref(p)) == 0, rq.lib().rfxq_last_error()
+    return p
+
+
 @pytest.mark.parametrize("ty,n,k,rows,few", [
     # measured, 32-row tiles -> few-row kernel (us): 20 -> 25, 20 -> 31, 19 -> 25, 56 -> 65, 31 -> 41, 30 -> 37, 35 -> 42
     (Q4K, 65280, 1024, 16, False), (Q4K, 65280, 1024, 32, False), (Q4K, 49152, 1024, 24, False),
@@ -212,9 +225,7 @@ def test_workspace_of_few_rows_fits_the_scratch(rq, ty, n, k, rows):
 def test_few_row_kernel_is_used_where_it_is_faster(rq, ty, n, k, rows, few):
     """Up to a 256-column tile per CU: the few-row kernel's ranges need workspace for their partials, the unsplit
     tiles for the f16 layout of the rows only (a 16384 x 2048 matrix splits K either way)."""
-    import torch
-    w = rq.Weight(rq.GgmlType(ty), torch.empty(16, dtype=torch.uint8), [k, n])
-    assert (rq.gemm_workspace_size(w, rows) >= 2 * rows * n * 4) == few
+    assert (rq.gemm_workspace_size(_shape(rq, ty, n, k), rows) >= 2 * rows * n * 4) == few
 
 
 @pytest.mark.parametrize("ty,n,k,rows,n128", [
@@ -225,13 +236,28 @@ def test_few_row_kernel_is_used_where_it_is_faster(rq, ty, n, k, rows, few):
     (Q4K, 8430, 4096, 128, True), (Q6K, 8430, 4096, 33, True), (Q8_0, 8430, 4096, 33, True),
     (Q8_0, 14336, 14336, 48, True), (Q4K, 4096, 4096, 512, True)])
 def test_64x128_tiles_are_used_where_they_are_faster(rq, ty, n, k, rows, n128):
-    """GEMMs whose larger tiles split K: their plan's workspace holds the policy's partial sums, the 64 x 128 tiles'
-    fewer."""
-    import torch
-    w = rq.Weight(rq.GgmlType(ty), torch.empty(16, dtype=torch.uint8), [k, n])
-    p = rq.gemm_policy(ty, k, n, rows)
-    assert p["splits"] > 1
-    assert (rq.gemm_workspace_size(w, rows) < p["splits"] * rows * n * 4) == n128
+    """GEMMs whose larger tiles split K."""
+    w = _shape(rq, ty, n, k)
+    assert rq.gemm_policy(ty, k, n, rows)["splits"] > 1
+    p = _plan_policy(rq, w, rows)
+    assert ((p.tile_m, p.tile_n) == (64, 128)) == n128
+
+
+@pytest.mark.parametrize("ty", [Q4K, Q6K, Q8_0])
+@pytest.mark.parametrize("n,k", [(4096, 4096), (1024, 4096), (4096, 14336)])
+def test_workspace_holds_the_policys_plan(rq, ty, n, k):
+    """A workspace holds the policy's partial sums where the GEMM runs on tiles that need fewer, so that one sized for
+    the most rows a caller will have still holds the longer splits of fewer rows (as it did when every GEMM ran the
+    policy's plan)."""
+    w = _shape(rq, ty, n, k)
+    fewer = 0
+    for rows in (16, 33, 64, 100, 200, 333, 512, 1024):
+        p, q = rq.gemm_policy(ty, k, n, rows), _plan_policy(rq, w, rows)
+        for splits in (p["splits"], q.splits):
+            if splits > 1:
+                assert rq.gemm_workspace_size(w, rows) >= splits * rows * n * 4
+        fewer += q.splits < p["splits"]
+    assert fewer
 
 
 def test_policy_errors(rq):
