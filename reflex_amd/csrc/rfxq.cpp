@@ -2519,7 +2519,10 @@ int rfxq_gemm_gate_up_silu_q8_1(const void* act, uint32_t rows, const rfxq_weigh
     }
     // separate GEMMs into the workspace, then SiLU·up into y and act_out
     const uint64_t u_bytes = align256((uint64_t)rows * ffn * 4u);
-    const uint64_t need = rfxq_gemm_gate_up_silu_workspace_size(gate, rows);
+    uint64_t need = rfxq_gemm_gate_up_silu_workspace_size(gate, rows);
+    // where that is not there, as much as the policy's plans need (as rfxq_gemm)
+    if (workspace ? workspace_bytes < need : !ws_available(c, need, stream))
+        need = 2u * u_bytes + plan_gemm(c, gate, std::max(rows, 2u), o, false, true).total;
     void* ws = workspace;
     if (!ws) {
         if (int rc = ctx_workspace(c, need, &ws, stream)) return rc;

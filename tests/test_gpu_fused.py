@@ -166,3 +166,31 @@ def test_gemm_gate_up_silu_q8_1(rq, orc, opts, ty, rows, ffn, k):
         with np.errstate(over="ignore"):
             ref = gr / (1.0 + np.exp(-gr)) * ur
         assert orc.rel_err_row_l2(got_y.cpu().numpy().reshape(rows, ffn), ref) < 1e-3
+
+
+def test_gate_up_silu_in_the_policys_workspace(rq, opts):
+    """The separate form in a workspace that holds the policy's plan only (no partial sums: 129 column tiles run
+    unsplit), where the few-row kernel would split K in two: accepted, on the policy's tiles. Both cut the same
+    sums of four super-blocks, each rounded within 2^-23 of the sum of magnitudes."""
+    rows, ffn, k = 16, 33024, 1024
+    one = synth.weights(Q6K, 258, k, 61).reshape(258, -1)
+    g = rq.Weight(rq.GgmlType(Q6K), _dev(np.tile(one[:129], (256, 1)).reshape(-1)), [k, ffn])
+    u = rq.Weight(rq.GgmlType(Q6K), _dev(np.tile(one[129:], (256, 1)).reshape(-1)), [k, ffn])
+    L = rq.lib()
+    size = L.rfxq_gemm_gate_up_silu_workspace_size
+    full = size(g.cref(), rows)
+    with rq.options(quant_mma_splits=1):
+        small = size(g.cref(), rows)
+    assert small < full
+    act = rq.quantize_act_q8_1(_dev(synth.activations(rows * k, 62)), rows, k)
+    _, want = rq.gemm_gate_up_silu_q8_1(act, rows, g, u)
+    got, out = torch.empty_like(want), torch.empty(rq.act_q8_1_size(rows, ffn), dtype=torch.uint8, device=DEV)
+    ws = torch.empty(small, dtype=torch.uint8, device=DEV)
+
+    def run(n):
+        return L.rfxq_gemm_gate_up_silu_q8_1(act.data_ptr(), rows, g.cref(), u.cref(), out.data_ptr(), got.data_ptr(),
+                                             ws.data_ptr(), n, torch.cuda.current_stream().cuda_stream)
+
+    assert run(small) == 0, L.rfxq_last_error()
+    assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max())
+    assert run(small - 256) == 11
