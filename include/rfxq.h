@@ -265,7 +265,7 @@ int rfxq_rmsnorm_q8_1(const float* x, const float* weight, uint32_t rows, uint32
 
 /* Model::silu_and_mul (src/kernels_cuda/silu_and_mul.cu:7-23) fused with the
  * quantization of its output (y optional, equal to rfxq_silu_and_mul's; it
- * must not alias gate or up, which are read once per layout). */
+ * must not alias gate or up, which may be read twice). */
 int rfxq_silu_and_mul_q8_1(const float* gate, const float* up, uint32_t rows, uint32_t k, void* act, float* y,
                            hipStream_t stream);
 

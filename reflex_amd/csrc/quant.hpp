@@ -471,24 +471,25 @@ struct QuantSrcSilu {
     }
 };
 
-extern "C" __global__ __launch_bounds__(1024) void rfxq_silu_and_mul_q8_1(const float* __restrict__ gate,
-                                                                        const float* __restrict__ up,
-                                                                        uint32_t rows, uint32_t k,
-                                                                        int8_t* __restrict__ xq,
-                                                                        uint32_t* __restrict__ xds,
-                                                                        uint16_t* __restrict__ xh,
-                                                                        uint16_t* __restrict__ xsx,
-                                                                        float* __restrict__ xrs,
-                                                                        float* __restrict__ y) {
-    const QuantSrcSilu src{gate, up, k};
-    for (uint32_t r = blockIdx.x; r < rows && xh; r += gridDim.x) {
-        if (xq) act_f16_row_wg<true, kActWgThreads>(src, r, k, xh, xsx, xrs, y, ActI8{xq, xds});
-        else act_f16_row_wg<false, kActWgThreads>(src, r, k, xh, xsx, xrs, y);
+// A row per workgroup of 1024 threads (up to a row per CU, or rows of more
+// than 4096 values) or 256 (more rows than CUs: 640 x 1536 7.2 us with 1024
+// threads, 7.1 with a row per wave, 5.2 with 256); the host's silu_form.
+#define RFXQ_SILU_ENTRY(NAME, NT)                                                                                \
+    extern "C" __global__ __launch_bounds__(NT) void NAME(                                                       \
+        const float* __restrict__ gate, const float* __restrict__ up, uint32_t rows, uint32_t k,                 \
+        int8_t* __restrict__ xq, uint32_t* __restrict__ xds, uint16_t* __restrict__ xh,                          \
+        uint16_t* __restrict__ xsx, float* __restrict__ xrs, float* __restrict__ y) {                            \
+        const QuantSrcSilu src{gate, up, k};                                                                     \
+        for (uint32_t r = blockIdx.x; r < rows && xh; r += gridDim.x) {                                          \
+            if (xq) act_f16_row_wg<true, NT>(src, r, k, xh, xsx, xrs, y, ActI8{xq, xds});                        \
+            else act_f16_row_wg<false, NT>(src, r, k, xh, xsx, xrs, y);                                          \
+        }                                                                                                        \
+        if (!xh && xq)                                                                                           \
+            quant_q8_1_rows(src, rows, k, xq, k, xds, y, ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6, \
+                            ((uint64_t)gridDim.x * blockDim.x) >> 6);                                            \
     }
-    if (!xh && xq)
-        quant_q8_1_rows(src, rows, k, xq, k, xds, y, ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6,
-                        ((uint64_t)gridDim.x * blockDim.x) >> 6);
-}
+RFXQ_SILU_ENTRY(rfxq_silu_and_mul_q8_1, 1024)
+RFXQ_SILU_ENTRY(rfxq_silu_and_mul_q8_1_256, 256)
 
 // the same with a row per wave (many short rows), the f16 layout at least
 extern "C" __global__ __launch_bounds__(256) void rfxq_silu_and_mul_q8_1_wave(

@@ -158,7 +158,7 @@ struct Ctx {
     hipFunction_t act_f16 = nullptr, act_f16_multi = nullptr, act_f16_wg = nullptr, act_f16_multi_wg = nullptr;
     hipFunction_t deq[3][2] = {};
     hipFunction_t gather = nullptr, scatter = nullptr, silu = nullptr, combine = nullptr;
-    hipFunction_t rms_q = nullptr, silu_q = nullptr, silu_q_wave = nullptr;
+    hipFunction_t rms_q = nullptr, silu_q = nullptr, silu_q_256 = nullptr, silu_q_wave = nullptr;
     hipFunction_t moe_route = nullptr, moe_route_w = nullptr, moe_plan = nullptr;
     // MoE decode kernels: [Q4_K, Q6_K, Q8_0][4, 8, 16, 32 lanes per row]
     hipFunction_t moe_dec_gu[3][4] = {}, moe_dec_dn[3][4] = {};
@@ -252,6 +252,7 @@ int load_ctx(int device, Ctx** out) {
         {&c->silu, "rfxq_silu_and_mul"},
         {&c->rms_q, "rfxq_rmsnorm_q8_1"},
         {&c->silu_q, "rfxq_silu_and_mul_q8_1"},
+        {&c->silu_q_256, "rfxq_silu_and_mul_q8_1_256"},
         {&c->silu_q_wave, "rfxq_silu_and_mul_q8_1_wave"},
         {&c->moe_route, "rfxq_moe_route"},
         {&c->moe_route_w, "rfxq_moe_route_w"},
@@ -1243,19 +1244,43 @@ int launch_quant(Ctx* c, const float* x, uint32_t ldx, const int32_t* src_rows, 
                   "rfxq_quantize_q8_1 launch");
 }
 
-// f16 layout of x (rfxq_act_f16): one wave per row
-// f16 activation kernels: a row per wave (rfxq_act_f16[_multi], 4 rows per
-// workgroup) for at least 128 rows of at most 4096 values, else a row per
-// workgroup (rfxq_act_f16[_multi]_wg: few rows, or rows too long for one
-// wave's registers)
+// Activation kernels: a row per wave (4 per workgroup) or a row per workgroup
+// (_wg: few rows, or rows too long for one wave's registers). A plan's f16
+// layouts (rfxq_act_f16_multi) run a row per wave from 128 rows of at most
+// 4096 values each.
 bool act_f16_wave(uint32_t rows, uint32_t k) { return k <= 4096u && rows >= 128u; }
 constexpr uint32_t kActWgThreads = 1024;  // of the row-per-workgroup kernels (quant.hpp)
-// The SiLU producers, a row per workgroup -> per wave (us): 4096 x 1024 30.5 ->
-// 14.9 (a quarter of the 1024 threads have values), 1024 x 1024 8.3 -> 6.2,
-// 2048 x 4096 24.7 -> 22.3; 1024 x 4096 17.7 per wave, 16.8 with 256 threads a row.
-bool silu_wave(uint32_t rows, uint32_t k) { return (k <= 2048u && rows >= 1024u) || (k <= 4096u && rows >= 2048u); }
+// Whether a row per wave is faster for `rows` rows in one launch: workgroups of
+// 1024 threads come in rounds of 256, whatever the row's length, while a
+// wave's time grows with it. Measured at 64-4096 rows of 256-4096 values, both
+// layouts of a row per workgroup -> per wave (us): 257 x 768 3.8 -> 3.6, 512 x
+// 512 4.5 -> 3.5, 512 x 2048 4.9 -> 5.6, 640 x 1280 6.2 -> 4.6, 1000 x 1024 7.5 -> 4.5.
+bool act_wave(uint32_t rows, uint32_t k) { return k <= 4096u && rows != 0u && k <= 640u * (uint64_t)((rows - 1u) / 256u); }
+// the same for one activation's layouts: from 1024 rows on a row per wave at any
+// K it holds (both layouts: 0.5-0.9 of the time, 1.03-1.10 at 1024-1280 x 4096)
+bool act_wave_one(uint32_t rows, uint32_t k) { return act_wave(rows, k) || (k <= 4096u && rows >= 1024u); }
 uint32_t act_f16_grid(uint32_t rows, bool wave) {
     return wave ? std::min<uint32_t>((rows + 3u) / 4u, 4096u) : std::min<uint32_t>(rows, 16384u);
+}
+
+// The SiLU producer's kernel: 1024 threads a row for up to a row per CU, a row
+// per wave for many short rows, 256 threads a row between (f16 layout written;
+// the int8 layout alone is spread over all waves). Measured over 1-4096 rows of
+// 256-6144 values, 1024 threads / a wave / 256 threads a row (us): 256 x 1024
+// 3.4 / 5.6 / 3.7; 512 x 1024 5.0 / 5.7 / 4.2; 640 x 1536 7.2 / 7.1 / 5.2; 1000 x
+// 256 7.8 / 3.8 / 5.4; 1000 x 1536 9.3 / 7.5 / 7.4; 1024 x 4096 14.8 / 17.7 / 13.0;
+// 2048 x 2048 19.3 / 13.1 / 14.1; 2048 x 4096 25.0 / 25.7 / 22.5; 4096 x 1024 29.9 /
+// 15.0 / 17.3.
+struct SiluForm {
+    hipFunction_t kernel;
+    uint32_t grid, threads;
+};
+SiluForm silu_form(const Ctx* c, uint32_t rows, uint32_t k, bool h) {
+    if (!h) return {c->silu_q, (quant_grid((uint64_t)rows * (k / 32u)) + 3u) / 4u, kActWgThreads};
+    if (rows <= (k > 3072u ? 512u : 256u) || k > 4096u) return {c->silu_q, act_f16_grid(rows, false), kActWgThreads};
+    const uint32_t wave_k = rows >= 2048u ? 3840u : rows > 1536u ? 2048u : rows > 768u ? 1280u : 0u;
+    if (k <= wave_k) return {c->silu_q_wave, act_f16_grid(rows, true), 256u};
+    return {c->silu_q_256, act_f16_grid(rows, false), 256u};
 }
 
 int launch_act_f16(Ctx* c, const float* x, uint32_t ldx, const int32_t* src_rows, uint32_t rows, uint32_t k,
@@ -1270,9 +1295,7 @@ int launch_act_f16(Ctx* c, const float* x, uint32_t ldx, const int32_t* src_rows
         float* xrs;
     } a = {x, ldx, 0, src_rows, rows, k, reinterpret_cast<uint16_t*>(base + L.xh),
            reinterpret_cast<uint16_t*>(base + L.xsx), reinterpret_cast<float*>(base + L.xrs)};
-    // (one activation: the row-per-wave kernel only once its grid fills the
-    // chip; 512 rows of 2048 take 6 us as 512 workgroups against 9.6 us as 128)
-    const bool wave = act_f16_wave(rows, k) && rows >= 1024u;
+    const bool wave = act_wave_one(rows, k);
     return launch(wave ? c->act_f16 : c->act_f16_wg, act_f16_grid(rows, wave), 0, stream, &a, sizeof a,
                   "rfxq_act_f16 launch", wave ? 256u : kActWgThreads);
 }
@@ -1292,7 +1315,7 @@ int launch_act(Ctx* c, const float* x, uint32_t rows, uint32_t k, uint8_t* base,
         } a = {x, rows, k, reinterpret_cast<int8_t*>(base + L.xq), reinterpret_cast<uint32_t*>(base + L.xds),
                reinterpret_cast<uint16_t*>(base + L.xh), reinterpret_cast<uint16_t*>(base + L.xsx),
                reinterpret_cast<float*>(base + L.xrs)};
-        const bool wave = act_f16_wave(rows, k) && rows >= 1024u;  // as launch_act_f16
+        const bool wave = act_wave_one(rows, k);
         return launch(wave ? c->act_both : c->act_both_wg, act_f16_grid(rows, wave), 0, stream, &a, sizeof a,
                       "rfxq_act_both launch", wave ? 256u : kActWgThreads);
     }
@@ -1330,10 +1353,8 @@ int launch_silu_act(Ctx* c, const float* gate, const float* up, uint32_t rows, u
            h ? reinterpret_cast<uint16_t*>(base + L.xsx) : nullptr,
            h ? reinterpret_cast<float*>(base + L.xrs) : nullptr,
            nullptr};
-    const bool wave = h && silu_wave(rows, k);
-    const uint32_t grid = h ? act_f16_grid(rows, wave) : (quant_grid((uint64_t)rows * (k / 32u)) + 3u) / 4u;
-    return launch(wave ? c->silu_q_wave : c->silu_q, grid, 0, stream, &a, sizeof a, "rfxq_silu_and_mul_q8_1 launch",
-                  wave ? 256u : kActWgThreads);
+    const SiluForm f = silu_form(c, rows, k, h);
+    return launch(f.kernel, f.grid, 0, stream, &a, sizeof a, "rfxq_silu_and_mul_q8_1 launch", f.threads);
 }
 
 // rfxq_moe_combine: out[t,:] = sum over the token's k pairs of w * pair_out row
@@ -2419,10 +2440,8 @@ int rfxq_silu_and_mul_q8_1(const float* gate, const float* up, uint32_t rows, ui
     } a = {gate, up, rows, k, reinterpret_cast<int8_t*>(b + L.xq), reinterpret_cast<uint32_t*>(b + L.xds),
            reinterpret_cast<uint16_t*>(b + L.xh), reinterpret_cast<uint16_t*>(b + L.xsx),
            reinterpret_cast<float*>(b + L.xrs), y};
-    const bool wave = silu_wave(rows, k);
-    if (int rc = launch(wave ? c->silu_q_wave : c->silu_q, act_f16_grid(rows, wave), 0, stream, &a, sizeof a,
-                        "rfxq_silu_and_mul_q8_1 launch", wave ? 256u : kActWgThreads))
-        return rc;
+    const SiluForm f = silu_form(c, rows, k, true);
+    if (int rc = launch(f.kernel, f.grid, 0, stream, &a, sizeof a, "rfxq_silu_and_mul_q8_1 launch", f.threads)) return rc;
     return ok();
 }
 
@@ -2631,9 +2650,18 @@ static int gemm_plan_create(const rfxq_gemm_item* items, uint32_t count, uint32_
         // one launch per layout kind for all activations
         std::vector<QuantDesc> q;
         std::vector<ActF16Desc> hq;
-        plan->hwave = true;  // one kernel for all f16 layouts: row per wave only if every activation allows it
-        for (const auto& a : plan->g.acts)
-            if (!a.ext && a.need_h && !act_f16_wave(rows, a.k)) plan->hwave = false;
+        // one kernel for all f16 layouts: a row per wave if every activation allows it, or where their rows
+        // together are many for the longest (64 activations of 64 x 1024: 40 -> 26 us with their GEMMs)
+        uint64_t hrows = 0;
+        uint32_t hk = 0;
+        plan->hwave = true;
+        for (const auto& a : plan->g.acts) {
+            if (a.ext || !a.need_h) continue;
+            if (!act_f16_wave(rows, a.k)) plan->hwave = false;
+            hrows += rows;
+            hk = std::max(hk, a.k);
+        }
+        plan->hwave |= act_wave((uint32_t)std::min<uint64_t>(hrows, 1u << 20), hk);
         for (const auto& a : plan->g.acts) {
             if (a.ext) continue;
             uint8_t* ab = base + a.off;

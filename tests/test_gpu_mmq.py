@@ -345,7 +345,9 @@ def test_gemm_few_rows_many_tiles(rq, ty, m, n, k):
     assert float((y - ref).abs().max()) <= 1e-5 * float(ref.abs().max())
 
 
-@pytest.mark.parametrize("rows,k", [(1024, 256), (1023, 2048), (1025, 2304), (2049, 4096), (3, 16640), (1024, 768)])
+@pytest.mark.parametrize("rows,k", [(1024, 256), (1023, 2048), (1025, 2304), (2049, 4096), (3, 16640), (1024, 768),
+                                    (256, 256), (257, 512), (257, 768), (513, 1280), (769, 1280),
+                                    (769, 1792), (1000, 512), (257, 4096), (2048, 4096), (2047, 3840)])
 def test_activation_producers_wave_and_workgroup(rq, rows, k):
     """The producers' layouts do not depend on how many rows a launch has (a row per wave or per workgroup,
     registers or two reads): the first and last row equal those of a one-row call, byte for byte."""
@@ -365,6 +367,23 @@ def test_activation_producers_wave_and_workgroup(rq, rows, k):
         first, last = parts(make(slice(0, k)), 1), parts(make(slice((rows - 1) * k, rows * k)), 1)
         for f, a, b in zip(full, first, last):
             assert torch.equal(f[0], a[0]) and torch.equal(f[1], b[0])
+
+
+@pytest.mark.parametrize("count,rows,k", [(9, 33, 512), (9, 33, 1024), (3, 100, 512), (2, 40, 4352)])
+def test_plan_of_many_short_activations(rq, orc, count, rows, k):
+    """A plan whose activations are short each and many together writes their f16 layouts a row per wave (297 rows
+    of 512: 9 x 33), else a row per workgroup: the bits of the single GEMMs on the same tiles."""
+    n = 130
+    with rq.options(quant_mma_splits=1):
+        items, want = [], []
+        for i in range(count):
+            x = _dev(synth.activations(rows * k, 1000 + i))
+            w = _weight(rq, Q4K, synth.weights(Q4K, n, k, 1020 + i), n, k)
+            items.append((x, w, torch.empty(rows * n, device=DEV)))
+            want.append(rq.gemm(x, w, rows))
+        rq.GemmPlan(items, rows).run()
+        for (_, _, y), ref in zip(items, want):
+            assert torch.equal(y, ref)
 
 
 def test_group_of_short_and_long_rows(rq, orc):
