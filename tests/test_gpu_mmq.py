@@ -310,9 +310,9 @@ def test_gemm_weight_past_4gib(rq, orc, ty):
 @pytest.mark.parametrize("ty", [Q4K, Q6K, Q8_0])
 @pytest.mark.parametrize("m,n,k", [(5, 70, 256), (16, 257, 2304), (17, 255, 1280), (32, 600, 4864), (9, 513, 14336)])
 def test_gemm_few_rows_kernel(rq, orc, ty, m, n, k):
-    """The few-row kernel at its edges: ragged column tiles, ranges of 1 to 8 super-blocks (16 rows)
-    and of 4 (17 rows up), a short last range; weights 2 bytes past a dword; an activation buffer instead of f32
-    rows; and an output over its own input, which takes the tile kernels."""
+    """The few-row kernel on ragged column tiles in ranges of one super-block (so few columns leave CUs for a
+    workgroup per super-block; longer ranges below); weights 2 bytes past a dword; an activation buffer instead of
+    f32 rows; and an output over its own input, which takes the tile kernels."""
     w_np = synth.weights(ty, n, k, 900 + m)
     x_np = synth.activations(m * k, 901 + m).reshape(m, k)
     y, _ = _check_gemm(rq, orc, ty, m, n, k, w_np, x_np)
@@ -327,6 +327,75 @@ def test_gemm_few_rows_kernel(rq, orc, ty, m, n, k):
         over = x.clone()
         got = rq.gemm(over, w, m, out=over)[:m * n].cpu().numpy().reshape(m, n)
         assert np.abs(got - y).max() <= 1e-5 * np.abs(y).max()
+
+
+@pytest.mark.parametrize("ty", [Q4K, Q6K, Q8_0])
+@pytest.mark.parametrize("m,k,splits,sb", [
+    (16, 2048, 1, 8),       # 70 KB of LDS, as many as a range may take
+    (15, 2048, 1, 8),       # 65.6 KB: just over 64 KB
+    (13, 17 * 256, 3, 6),   # 6, 6, 5
+    (9, 1280, 1, 5), (5, 1792, 1, 7),
+    (8, 17 * 256, 6, 3),    # 3 and a last range of 2
+    (17, 1024, 1, 4), (32, 1024, 1, 4),  # as many as 17 to 32 rows may take
+    (29, 7 * 256, 2, 4),    # 4 and 3
+    (24, 512, 1, 2)])
+def test_gemm_few_rows_long_ranges(rq, orc, opts, ty, m, k, splits, sb):
+    """The few-row kernel in ranges of 2 to 8 super-blocks, which stream (the next super-block's weights are in
+    flight while one is used), with short last ranges; up to 16 rows the staging holds 4 rows a wave of 8
+    super-blocks, and in ranges of up to 4 (17 to 32 rows) 8 rows of 4. Then weights 2 bytes past a dword and an
+    activation buffer, whose row scale changes no f16-normal value's rounding: the same bits."""
+    opts(quant_mma_splits=splits)
+    n = 257
+    p = rq.gemm_policy(ty, k, n, m)
+    assert (p["tile_m"], p["splits"], p["sb_per_split"]) == (32, splits, sb)
+    w_np = synth.weights(ty, n, k, 940 + m)
+    x_np = synth.activations(m * k, 941 + m).reshape(m, k)
+    y, _ = _check_gemm(rq, orc, ty, m, n, k, w_np, x_np)
+    act = rq.quantize_act_q8_1(_dev(x_np), m, k)
+    assert np.array_equal(rq.gemm_q8_1(act, _weight(rq, ty, w_np, n, k), m).cpu().numpy().reshape(m, n), y)
+    if ty != Q4K:
+        buf = torch.zeros(w_np.size + 16, dtype=torch.uint8, device=DEV)
+        buf[2:2 + w_np.size] = _dev(w_np)
+        w2 = rq.Weight(rq.GgmlType(ty), buf, [k, n], offset=2, len=w_np.size)
+        assert np.array_equal(rq.gemm(_dev(x_np), w2, m).cpu().numpy().reshape(m, n), y)
+        assert np.array_equal(rq.gemm_q8_1(act, w2, m).cpu().numpy().reshape(m, n), y)
+
+
+@pytest.mark.parametrize("ty", [Q4K, Q6K, Q8_0])
+def test_gemm_few_rows_scale_of_a_range(rq, orc, ty):
+    """Super-blocks 2^-26 apart (the large ones on zero weights): a range of one super-block scales the small ones
+    by their own maximum, an activation buffer by the row's, under which they are f16-subnormal. The f32 form keeps
+    the f16 kernels' error; the buffer's differs by half a subnormal step of the row's scale, 2^(e - 25) a value, at
+    the most (and the two forms' f16 and f32 roundings, 2^-10 of the magnitudes)."""
+    m, n, k = 12, 300, 2048
+    nsb = k // 256
+    w_np = synth.weights(ty, n, k, 950).reshape(n, nsb, -1).copy()
+    w_np[:, 0::2] = 0
+    w_np = w_np.reshape(-1)
+    x = synth.activations(m * k, 951).reshape(m, nsb, 256)
+    x[:, 1::2] *= np.float32(2.0 ** -26)
+    x = np.ascontiguousarray(x.reshape(m, k))
+    y = rq.gemm(_dev(x), _weight(rq, ty, w_np, n, k), m).cpu().numpy().reshape(m, n)
+    assert orc.rel_err_row_l2(y, orc.reference_gemm(ty, w_np, n, k, x)) < TOL
+    act = rq.quantize_act_q8_1(_dev(x), m, k)
+    yb = rq.gemm_q8_1(act, _weight(rq, ty, w_np, n, k), m).cpu().numpy().reshape(m, n)
+    aw = np.abs(orc.dequant_matrix(ty, w_np, n, k)).astype(np.float64)
+    step = 2.0 ** (np.ceil(np.log2(np.abs(x).max(axis=1, keepdims=True))) - 8 - 25)
+    bound = step * aw.sum(axis=1)[None] + 2.0 ** -10 * (np.abs(x).astype(np.float64) @ aw.T)
+    assert (np.abs(yb.astype(np.float64) - y) <= bound).all()
+
+
+@pytest.mark.parametrize("ty", [Q4K, Q6K, Q8_0])
+@pytest.mark.parametrize("m,tile_m", [(33, 64), (48, 64), (64, 64), (65, 128), (129, 128), (225, 128)])
+def test_gemm_row_counts_of_larger_tiles(rq, orc, opts, ty, m, tile_m):
+    """64 x 256 and 128 x 256 tiles at ragged row counts (a forced split keeps them where 64 x 128 tiles would run)."""
+    opts(quant_mma_splits=2)
+    n, k = 200, 1024
+    p = rq.gemm_policy(ty, k, n, m)
+    assert (p["tile_m"], p["tile_n"], p["splits"]) == (tile_m, 256, 2)
+    w_np = orc.synthetic(ty, k, n, 70 + m)
+    x = synth.activations(m * k, 71 + m).reshape(m, k)
+    _check_gemm(rq, orc, ty, m, n, k, w_np, x)
 
 
 @pytest.mark.parametrize("ty", [Q4K, Q6K, Q8_0])
