@@ -112,9 +112,11 @@ int rfxq_set_options(const rfxq_options* options);
  * quant_mma_max_rows (kernels.rs:628-713) and the fused-GEMV crossover
  * (:2144-2169), re-derived for MI355X; `compute_units` as the device reports.
  * tile and splits are the general plan's. Unless REFLEX_QUANT_MMA_SPLITS
- * forces a count, a GEMM of more than 32 rows may run on 64 x 128 tiles with
- * fewer ranges instead, where that is estimated faster; the sum over K is then
- * cut at other places. */
+ * forces a count, an f16 GEMM of up to 32 rows may run on the few-row kernel
+ * with other ranges, and one of more rows on 64 x 128 tiles with fewer ranges,
+ * where that is estimated faster and the workspace holds it; the sum over K is
+ * then cut at other places (also between an eager call and a captured one
+ * whose library workspace cannot grow). */
 typedef struct rfxq_gemm_policy {
     uint32_t path;
     uint32_t tile_m, tile_n;
@@ -201,7 +203,7 @@ int rfxq_gemm(const float* x, uint64_t x_len, const rfxq_weight* w, uint32_t row
 /* rfxq_gemm with no device allocation, for callers that cannot allocate
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc). It has no counterpart in the reference. Same path, kernels and
- * results as rfxq_gemm with a NULL workspace; the workspace is a fixed
+ * results as rfxq_gemm with a NULL workspace that can grow; the workspace is a fixed
  * 128 MiB device array per GPU (a file-scope __device__ array, held until the
  * process ends), so GEMMs that need more than it holds on every plan fail
  * with RFXQ_ERR_INVALID_INPUT. The device must be initialised first

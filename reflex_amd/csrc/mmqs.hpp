@@ -8,11 +8,14 @@
 // (all rows of the range) it holds in LDS as f16, so the loop over the range
 // has no barrier and no activation copies: each wave streams its own columns'
 // raw blocks into registers a whole super-block (9-17 KB a wave) ahead of
-// their use. The activations come straight from f32 (each workgroup converts
+// their use (ranges of one super-block, which a narrow matrix is cut into, ask
+// for theirs once and wait). The activations come straight from f32 (each workgroup converts
 // its range: no activation launch; a row's power-of-two scale is then the
-// range's, which changes no product's rounding) or from the f16 layout
-// (quant.hpp). Operands and the order of additions are the tile kernels'
-// (mmqh.hpp), so the results are theirs for the same split of K.
+// range's, under which no value keeps fewer bits, and those that the row's scale
+// would make f16-subnormal keep more) or from the f16 layout (quant.hpp).
+// Operands and the order of additions are the tile kernels' (mmqh.hpp), so for
+// the same split of K the results are theirs where the row's scale leaves every
+// value f16-normal (or zero).
 #pragma once
 #include "common.hpp"
 #include "mmq.hpp"
@@ -120,7 +123,7 @@ struct W4 {  // Q4_K
     u4_t q[2][2][2], h[2];  // raw: [stage pair][j][load A, B], headers
     u4_t dsc[2], cop[2];
     u4_t cur[2][4];  // the stages' operands bytes (after the lane swap)
-    uint32_t sm[2][2], mlo, mhi, mg;
+    uint32_t mlo, mhi, mg;
     RFXQ_MEMBER void init() {
         mlo = 0x000F000Fu, mhi = 0x00F000F0u, mg = 0x64006400u;
         asm("" : "+v"(mlo), "+v"(mhi), "+v"(mg));

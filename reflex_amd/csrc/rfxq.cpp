@@ -1480,7 +1480,8 @@ GemmPlan plan_gemm(const Ctx* c, const rfxq_weight* w, uint32_t rows, const rfxq
     p.off_part = p.act.total;
     p.total = p.off_part + (p.pol.splits > 1 ? align256((uint64_t)p.pol.splits * rows * n * 4u) : 0u);
     // more partials than the fixed scratch holds: the policy's plan if that
-    // needs less (one rule for every entry point, so that all give one result)
+    // needs less (at every entry point, so that all give one result; a call
+    // whose workspace is short of the plan runs the policy's too, `general`)
     if (sb && p.total > rfxq_scratch::kScratchBytes) {
         const GemmPlan g = plan_gemm(c, w, rows, o, in_place, true);
         if (g.total < p.total) return g;

@@ -4,7 +4,8 @@ them. Parity: the producers' f32 outputs are bit-identical to the reference
 kernels' (rmsnorm.cu through the oracle restatement; silu_and_mul.cu through
 rfxq_silu_and_mul), their activation buffers equal the quantizer's on those
 outputs byte for byte, and GEMMs from the buffers equal rfxq_gemm on the f32
-activations bit for bit."""
+activations bit for bit (where no value is f16-subnormal under its row's scale:
+the few-row kernel scales f32 rows by range)."""
 import numpy as np
 import pytest
 import torch
