@@ -1027,23 +1027,31 @@ uint32_t small_gemm_tile_m(uint32_t tile_m, uint32_t rows, uint32_t n, uint32_t 
 // ---- 64 x 128 tiles instead of the larger ones
 //
 // Estimated time (us, less what all tiles take alike) of one f16 launch of
-// GEMMs {n, super-blocks per row} of `rows` rows on `bm` x `bn` tiles with
-// ranges of `sb` super-blocks and the tiles' constants c. The launch ends with
+// GEMMs {n, super-blocks per row} of `rows` rows on tiles of `bn` columns, cut
+// as ts says, with the tiles' constants c. The launch ends with
 // its slowest XCD (each takes an eighth of the tiles, contiguous ones), whose
 // workgroups come to its CUs in rounds of one per CU: a launch of a few more
 // than a round ends a whole workgroup later (14336 x 4096 Q8_0 at 400 rows: 784
 // tiles of 64 x 128, four rounds, 169 us; 106 us as 224 of 128 x 256). A longer
 // workgroup than the XCD's mean ends late by as much more as there are fewer
-// rounds. Partial sums of split GEMMs are written and read once.
+// rounds. Partial sums of split GEMMs are written and read once. Unsplit results
+// whose rows are not whole 64-byte pieces leave parts of them at both ends of a
+// tile's rows, which the 256-column tiles store at half the rate (122059 x 256
+// Q6_K at 661 rows: 309 us on 128 x 256 tiles, 191 on 64 x 128).
 struct GemmShape {
     uint32_t n, nsb;
 };
-struct MmqhCost {
-    // us: fixed, per MB of partials, per super-block of an XCD's rounds, of its CUs' load, of the mean workgroup
-    double fixed, part, round, load, mean;
+// rows of a tile and super-blocks of the ranges that GEMMs of rows over `over` super-blocks are cut into
+struct TileSplit {
+    uint32_t tile_m, sb, over;
 };
-double mmqh_time(const std::vector<GemmShape>& g, uint32_t rows, uint32_t bm, uint32_t bn, uint32_t sb,
-                 const MmqhCost& c, uint32_t cus) {
+struct MmqhCost {
+    // us: fixed, per MB of partials, per super-block of an XCD's rounds, of its CUs' load, of the mean workgroup,
+    // per round, per MB of results in rows of broken 64-byte pieces
+    double fixed, part, round, load, mean, wg, line;
+};
+double mmqh_time(const std::vector<GemmShape>& g, uint32_t rows, uint32_t bn, TileSplit ts, const MmqhCost& c,
+                 uint32_t cus) {
     struct Run {
         uint64_t wgs;
         double mean;  // super-blocks
@@ -1051,17 +1059,25 @@ double mmqh_time(const std::vector<GemmShape>& g, uint32_t rows, uint32_t bm, ui
     };
     std::vector<Run> runs;
     uint64_t wgs = 0;
-    double total = 0.0, part = 0.0;
+    double total = 0.0, part = 0.0, line = 0.0;
+    bool sorted = false;  // a large launch that splits some rows starts the longest ranges first
     for (const auto& s : g) {
-        const uint64_t tiles = (uint64_t)((rows + bm - 1u) / bm) * ((s.n + bn - 1u) / bn);
-        const uint32_t splits = (s.nsb + sb - 1u) / sb;
+        const uint64_t tiles = (uint64_t)((rows + ts.tile_m - 1u) / ts.tile_m) * ((s.n + bn - 1u) / bn);
+        uint32_t splits = s.nsb > ts.over ? (s.nsb + ts.sb - 1u) / ts.sb : 1u;
+        if (ts.over) {
+            const uint32_t range = (s.nsb + splits - 1u) / splits;
+            splits = (s.nsb + range - 1u) / range;
+            sorted |= splits > 1u;
+        }
         runs.push_back({tiles * splits, (double)s.nsb / splits, (s.nsb + splits - 1u) / splits});
         wgs += tiles * splits;
         total += (double)tiles * s.nsb;
         if (splits > 1u) part += 8e-6 * splits * rows * s.n;
+        else if (s.n % 16u) line += 4e-6 * rows * s.n;
     }
+    if (sorted) std::stable_sort(runs.begin(), runs.end(), [](const Run& a, const Run& b) { return a.longest > b.longest; });
     const uint64_t xcd_cus = std::max(1u, cus / 8u);
-    double rounds = 0.0, load = 0.0;
+    double rounds = 0.0, load = 0.0, wg = 0.0;
     size_t at = 0;
     for (uint32_t x = 0; x < 8u; x++) {
         const uint64_t n = wgs / 8u + (x < wgs % 8u ? 1u : 0u);
@@ -1082,25 +1098,25 @@ double mmqh_time(const std::vector<GemmShape>& g, uint32_t rows, uint32_t bm, ui
         const double r = (double)((n + xcd_cus - 1u) / xcd_cus), mean = sum / n;
         rounds = std::max(rounds, r * mean + (longest - mean) / r);
         load = std::max(load, sum / xcd_cus);
+        wg = std::max(wg, r);
     }
-    return c.fixed + c.part * part + c.round * rounds + c.load * load + c.mean * total / wgs;
+    return c.fixed + c.part * part + c.round * rounds + c.load * load + c.mean * total / wgs + c.wg * wg + c.line * line;
 }
 
 // Super-blocks per range on 64 x 128 tiles for the GEMMs of one type and one
-// launch, or 0 where they are not estimated 4% (10%: 32-row tiles) faster than the larger tiles
-// `base` {rows, super-blocks per range}. 64 x 128 tiles split K only as far as
-// there are idle CUs. The constants are fitted to the measured differences of
-// 2550 single GEMMs (n 64-14336, K 256-14336, 33-1500 rows) and 2604 groups
-// (parts of a layer to eight layers, 33-1024 rows): the choices run 1.25x and
-// 1.13x faster than the larger tiles on average, 0.3% behind the faster of the
-// two; 52 are over 3% slower, 12% at the most but for two groups (20-24%). Main
+// launch, or 0 where they are not estimated 5% (10%: 32-row tiles) faster than
+// the larger tiles `base`. 64 x 128 tiles split K only as far as there are idle
+// CUs. The constants are fitted to the measured differences of 10000 single
+// GEMMs (n 64-151936, K 256-14336, 33-1500 rows) and 5500 groups (parts of a
+// layer, 33-1024 rows). Over 4000 other GEMMs and 2500 groups the choices run
+// 1.21x and 1.26x faster than the larger tiles on average, 0.25% behind the
+// faster of the two (groups ahead: two launches may choose apart): 32 and 12 are
+// over 3% slower than the larger tiles, 19% at the most, and 100 and 69 more
+// over 3% slower than 64 x 128 tiles would be. Main
 // launch and reduce at 4096 x 4096 Q4_K: 64 rows 11.5 + 3.5 -> 8.1 + 3.5 us,
 // 128 rows 15.2 + 4.5 -> 10.9 + 3.5, 512 rows 30.6 + 15.5 -> 28.6 + 0, 1024
 // rows 42.9 + 10 -> 50.2 + 0; 4096 x 14336 Q6_K at 512 rows stays on 128 x 256
 // tiles (92 + 15 against 123).
-struct TileSplit {
-    uint32_t tile_m, sb;
-};
 // Ranges no longer than the launch's shortest row: each XCD takes contiguous
 // tiles, and a GEMM of longer ones would keep its XCD busy alone (a Q8_0 8B
 // layer, K = 4096 and 14336: 198 us at 64 rows, 120 on 64 x 256 tiles, now
@@ -1119,17 +1135,17 @@ uint32_t n128_split(const std::vector<std::pair<uint32_t, uint32_t>>& tiles_nsb,
 uint32_t n128_sb(const std::vector<GemmShape>& g, uint32_t ty, uint32_t rows, uint32_t cus, TileSplit base) {
     // [type][128 x 256, 64 x 256, 32 x 256, 64 x 128]
     static const MmqhCost kCost[3][4] = {
-        {{2.2, 0.23, 2.36, 0.88, 0.57}, {0.27, 0.27, 1.8, 0.53, 0.67}, {0.39, 0.2, 0.93, 0.73, 0.37}, {0, 0.27, 0.68, 0.54, 0.49}},
-        {{2.57, 0.22, 4.3, 0.058, 0.61}, {1.2, 0.3, 3.6, 0.36, 0}, {-1.33, 0.36, 3.03, 0, 1.07}, {0, 0.31, 1.66, 0.43, 0.04}},
-        {{3.58, 0.23, 4.01, 0, 0.82}, {0.82, 0.32, 4.09, 0.19, 0}, {-0.33, 0.3, 2.23, 0, 1.71}, {0, 0.29, 1.77, 0.043, 0.39}}};
+        {{1.06, 0.179, 2.21, 0.837, 0.457, 0.841, 0.142}, {0.721, 0.211, 1.33, 0.762, 0.685, 0.243, 0}, {0.446, 0.209, 0.873, 0.778, 0.365, 0, 0}, {0, 0.246, 0.619, 0.514, 0.36, 0.124, 0}},
+        {{0.887, 0.16, 3.33, 1.04, 0.613, 3.54, 0.234}, {-0.0173, 0.224, 3.05, 0.848, 0, 2.84, 0.12}, {-0.461, 0.373, 2.09, 0, 2.2, 0, 0.212}, {0, 0.233, 1.73, 0.196, 0.168, 1.37, 0}},
+        {{0, 0.167, 3.14, 1, 1.26, 2.75, 0.213}, {-0.981, 0.229, 3.39, 0.79, 0, 2.06, 0.116}, {-0.585, 0.302, 1.57, 0, 1.92, 0, 0.14}, {0, 0.238, 1.62, 0.123, 0.12, 0.364, 0}}};
     if (rows <= 32u) return 0u;
     const int t = type_index(ty);
     std::vector<std::pair<uint32_t, uint32_t>> tiles;
     for (const auto& s : g) tiles.push_back({((rows + 63u) / 64u) * ((s.n + 127u) / 128u), s.nsb});
     const uint32_t sb = n128_split(tiles, cus);
     const int b = base.tile_m >= 128u ? 0 : base.tile_m == 64u ? 1 : 2;
-    const double big = mmqh_time(g, rows, base.tile_m, 256u, base.sb, kCost[t][b], cus);
-    return mmqh_time(g, rows, 64u, 128u, sb, kCost[t][3], cus) < (b == 2 ? 0.9 : 0.96) * big ? sb : 0u;
+    const double big = mmqh_time(g, rows, 256u, base, kCost[t][b], cus);
+    return mmqh_time(g, rows, 128u, {64u, sb, 0u}, kCost[t][3], cus) < (b == 2 ? 0.9 : 0.95) * big ? sb : 0u;
 }
 
 // raw bytes of a weight matrix
@@ -1463,7 +1479,7 @@ GemmPlan plan_gemm(const Ctx* c, const rfxq_weight* w, uint32_t rows, const rfxq
             sb = std::min(split_sb({{tiles, nsb}}, 1u, 2u * std::max(cus, 1u)), few_max_sb(rows));
         }
     } else if (p.f16 && !general && !forced) {
-        sb = n128_sb({{n, nsb}}, w->ggml_type, rows, cus, {p.pol.tile_m, p.pol.sb_per_split});
+        sb = n128_sb({{n, nsb}}, w->ggml_type, rows, cus, {p.pol.tile_m, p.pol.sb_per_split, 0u});
         if (sb) {
             p.n128 = true;
             p.pol.tile_m = 64u;
@@ -1705,7 +1721,7 @@ int build_gemm_group(const rfxq_gemm_item* items, uint32_t count, uint32_t rows,
     for (uint32_t t = 6u; t < kGroupFew && !o.quant_mma_splits && !general; t++) {
         std::vector<GemmShape> shapes;
         std::vector<std::pair<uint32_t, uint32_t>> tn, by_sb;
-        uint32_t ty = 0, tiles = 0, max_nsb = 0;
+        uint32_t ty = 0, tiles = 0;
         for (uint32_t i = 0; i < count; i++) {
             if (item_act[i] == ~0u || item_kernel[i] != t) continue;
             ty = items[i].w->ggml_type;
@@ -1714,12 +1730,15 @@ int build_gemm_group(const rfxq_gemm_item* items, uint32_t count, uint32_t rows,
             tn.push_back({((rows + bm - 1u) / bm) * ((shapes.back().n + 255u) / 256u), shapes.back().nsb});
             tiles += tn.back().first;
             by_sb.push_back({shapes.back().nsb, tn.back().first});
-            max_nsb = std::max(max_nsb, shapes.back().nsb);
         }
         if (shapes.empty()) continue;
-        const uint32_t med = median_sb(by_sb);  // (the larger tiles split rows over 3x it, below)
-        const uint32_t sb = 2u * tiles < cus ? split_sb(tn, 2u, 2u * std::max(cus, 1u)) : max_nsb > 3u * med ? med : max_nsb;
-        if (n128_sb(shapes, ty, rows, cus, {group_tile_m(t), sb}))
+        // as the larger tiles are split below: all rows of a small launch, rows over 3x the median of a large one
+        TileSplit base{group_tile_m(t), split_sb(tn, 2u, 2u * std::max(cus, 1u)), 0u};
+        if (2u * tiles >= cus) {
+            base.sb = median_sb(by_sb);
+            base.over = shapes.size() > 1u ? 3u * base.sb : base.sb;
+        }
+        if (n128_sb(shapes, ty, rows, cus, base))
             for (uint32_t i = 0; i < count; i++)
                 if (item_act[i] != ~0u && item_kernel[i] == t) item_kernel[i] = kGroupN128 + (uint32_t)type_index(ty);
     }

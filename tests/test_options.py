@@ -243,6 +243,18 @@ def test_64x128_tiles_are_used_where_they_are_faster(rq, ty, n, k, rows, n128):
     assert ((p.tile_m, p.tile_n) == (64, 128)) == n128
 
 
+@pytest.mark.parametrize("ty,n,k,rows,n128", [
+    # measured, larger tiles -> 64 x 128 (us): 309 -> 191, 246 -> 165, 187 -> 117, 88 -> 71; 91 -> 76
+    (Q6K, 122059, 256, 661, True), (Q8_0, 98852, 256, 870, True), (Q4K, 123699, 512, 447, True),
+    (Q8_0, 14487, 1792, 519, True), (Q8_0, 21774, 768, 795, True),
+    # rows of whole lines: 21 -> 27, 86 -> 94
+    (Q8_0, 111360, 256, 70, False)])
+def test_64x128_tiles_where_rows_are_not_whole_lines(rq, ty, n, k, rows, n128):
+    """Unsplit GEMMs: results in rows that are not whole 128-byte lines cost the 256-column tiles more."""
+    p = _plan_policy(rq, _shape(rq, ty, n, k), rows)
+    assert ((p.tile_m, p.tile_n) == (64, 128)) == n128
+
+
 @pytest.mark.parametrize("ty", [Q4K, Q6K, Q8_0])
 @pytest.mark.parametrize("n,k", [(4096, 4096), (1024, 4096), (4096, 14336)])
 def test_workspace_holds_the_policys_plan(rq, ty, n, k):
