@@ -918,22 +918,30 @@ uint32_t few_max_sb(uint32_t rows) { return rows > 32u ? 0u : rows > 16u ? 4u : 
 uint32_t few_lds(uint32_t rows, uint32_t sb) {
     return 128u + std::max(16384u, rows * (sb * 544u + 16u));  // (results pass through 4 KB per wave)
 }
-// Whether one launch of 32 x 256 tiles runs on the few-row kernel. It keeps more weight bytes in flight than the 32-row tiles,
-// but each of its workgroups brings the f32 rows in itself, and its short
-// ranges write more partials: both grow with the rows.
-// - Tiles for less than half the CUs: the tiles split K as well, and the
-//   few-row kernel is faster but for many rows of long launches (an 8B layer,
-//   3300 super-blocks: 24 rows 78 -> 74 us, 32 rows 78 -> 79).
+// Whether one launch of 32 x 256 tiles runs on the few-row kernel. It keeps
+// more weight bytes in flight than the 32-row tiles, but each of its workgroups
+// brings the f32 rows in itself, and its short ranges write more partials: both
+// grow with the rows.
+// - Tiles for less than half the CUs: the tiles split K as well, and the few-row
+//   kernel is faster (0.86 of their time) unless more than 12 Q4_K rows are so
+//   long that its longest range cuts the launch into more than two workgroups a
+//   CU (22532 x 11008 at 15 rows 47 -> 58 us, 31828 x 8704 at 23 rows 52 -> 65;
+//   27092 x 14336 at 9 rows 85 -> 68; Q6_K 0.9-1.0 of the tiles' time there, Q8_0
+//   0.8-0.9).
 // - Up to a tile per CU: the tiles run unsplit, so their time is a whole row's
 //   whatever their number, and the few-row kernel's is its longest range (two
-//   workgroups a CU), its partials and its results. The constants (us: fixed,
+//   workgroups a CU), its partials and its results. The constants are us: fixed,
 //   per super-block of a row, per super-block of a range, per row and range of
-//   a CU, per row and tile of a CU) are fitted to 4100 launches of 129 to 256
-//   tiles (1 to 56 super-blocks, 5 to 32 rows). Of those and 2050 launches of
-//   fewer tiles 34 are over 3% slower for the choice, 8% at the most. Launches
-//   of one range a row write no partials and always win. At exactly half the CUs
-//   (the fewest tiles that run unsplit) they are slowest, hence its own line.
+//   a CU, per row and tile of a CU; the few-row kernel has to be 10% of a row's
+//   time ahead, but for exactly half the CUs (the fewest tiles that run unsplit:
+//   the slowest), where it may be 16% behind. Launches of one range a row write
+//   no partials and always win. A group of many rows stays on tiles (an 8B layer,
+//   3300 super-blocks: 24 rows 78 -> 74 us, 32 rows 78 -> 79).
 // - More tiles fill every CU.
+// Of 2500 launches of up to a tile per CU with their weights in memory (1 to 56
+// super-blocks, 5 to 32 rows) 22 are over 3% slower than the tiles for the choice,
+// 9% at the most, 0.4% behind the faster of the two on average; of 9840 with their
+// weights in the caches 172 over 3%, 17 over 10% (22% at the most), 0.25%.
 // Measured, 32-row tiles -> few-row kernel (us), Q4_K / Q6_K / Q8_0:
 //   4096 x 4096       16 rows 15 -> 12 / 18 -> 16 / 17 -> 15;   32: 17 -> 15 / 19 -> 18 / 19 -> 18
 //   32768 x 2048      16 rows 29 -> 23 / 45 -> 28 / 55 -> 38;   32: 30 -> 27 / 45 -> 34 / 56 -> 43
@@ -964,8 +972,6 @@ bool few_wins(const std::vector<FewShape>& gemms, uint32_t rows, uint32_t cus) {
         if (rows <= (q4k ? 8u : 16u)) return max_nsb > 4u || tiles >= 2u * cus;
         return !q4k && max_nsb <= 4u && tiles >= 2u * cus;  // (one range: no partials)
     }
-    if (rows > 24u && load > 8ull * cus) return false;
-    if (2u * tiles < cus) return true;
     static const double kCost[3][5] = {{2.4, 2.1, 2.4, 0.15, 0.15}, {2.6, 3.5, 4.0, 0.089, 0.22}, {4.0, 4.3, 5.3, 0.033, 0.33}};
     const uint32_t sb = std::min(split_sb(tn, 1u, 2u * std::max(cus, 1u)), few_max_sb(rows));
     uint64_t ranges = 0;
@@ -977,12 +983,13 @@ bool few_wins(const std::vector<FewShape>& gemms, uint32_t rows, uint32_t cus) {
         row_sum += kCost[g.type][1] * g.nsb * g.tiles;
         range_max = std::max(range_max, kCost[g.type][2] * ((g.nsb + s - 1u) / s));
     }
+    if (2u * tiles < cus) return !q4k || rows <= 12u || ranges <= 2ull * cus;
+    if (gemms.size() > 1u && rows > 24u && load > 8ull * cus) return false;
     if (ranges == tiles) return true;
-    if (2u * tiles == cus) return q4k ? rows <= 12u || load >= 8ull * tiles : rows <= 20u || load >= 4ull * tiles;
     const double* c = kCost[q4k ? 0 : gemms[0].type];
     const double rounds = (double)((ranges + 2u * cus - 1u) / (2u * cus));
     // (a group's tiles end between its longest row and the mean one)
-    return c[0] - 0.5 * (row_max + row_sum / tiles) + range_max * rounds + (c[3] * ranges + c[4] * tiles) * rows / cus < 0.0;
+    return c[0] - (2u * tiles == cus ? 0.58 : 0.45) * (row_max + row_sum / tiles) + range_max * rounds + (c[3] * ranges + c[4] * tiles) * rows / cus < 0.0;
 }
 
 // Row tile of one grouped MoE GEMM, `pairs` routed rows over `experts`

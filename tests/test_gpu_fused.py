@@ -171,9 +171,9 @@ def test_gemm_gate_up_silu_q8_1(rq, orc, opts, ty, rows, ffn, k):
 
 def test_gate_up_silu_in_the_policys_workspace(rq, opts):
     """The separate form in a workspace that holds the policy's plan only (no partial sums: 129 column tiles run
-    unsplit), where the few-row kernel would split K in two: accepted, on the policy's tiles. Both cut the same
-    sums of four super-blocks, each rounded within 2^-23 of the sum of magnitudes."""
-    rows, ffn, k = 16, 33024, 1024
+    unsplit), where the few-row kernel would split K: accepted, on the policy's tiles. Both cut the same
+    sums of eight super-blocks, each rounded within 2^-23 of the sum of magnitudes."""
+    rows, ffn, k = 16, 33024, 2048
     one = synth.weights(Q6K, 258, k, 61).reshape(258, -1)
     g = rq.Weight(rq.GgmlType(Q6K), _dev(np.tile(one[:129], (256, 1)).reshape(-1)), [k, ffn])
     u = rq.Weight(rq.GgmlType(Q6K), _dev(np.tile(one[129:], (256, 1)).reshape(-1)), [k, ffn])

@@ -218,6 +218,8 @@ def _plan_policy(rq, w, rows):
     (Q4K, 65280, 1024, 16, False), (Q4K, 65280, 1024, 32, False), (Q4K, 49152, 1024, 24, False),
     (Q4K, 65280, 4096, 24, False), (Q4K, 57344, 2048, 32, False), (Q6K, 61440, 1024, 32, False),
     (Q8_0, 65280, 1024, 24, False),
+    # 80 -> 93, 116 -> 138, 16 -> 19
+    (Q4K, 51510, 8192, 23, False), (Q6K, 59700, 5376, 24, False), (Q8_0, 33280, 768, 16, False),
     # 30 -> 27, 55 -> 44, 18 -> 15, 89 -> 76, 46 -> 40, 33 -> 28, 104 -> 72
     (Q4K, 32768, 2048, 32, True), (Q4K, 65280, 4096, 8, True), (Q4K, 16384, 2048, 5, True),
     (Q6K, 65280, 4096, 16, True), (Q6K, 40960, 2048, 32, True), (Q8_0, 32768, 1024, 32, True),
@@ -226,6 +228,22 @@ def test_few_row_kernel_is_used_where_it_is_faster(rq, ty, n, k, rows, few):
     """Up to a 256-column tile per CU: the few-row kernel's ranges need workspace for their partials, the unsplit
     tiles for the f16 layout of the rows only (a 16384 x 2048 matrix splits K either way)."""
     assert (rq.gemm_workspace_size(_shape(rq, ty, n, k), rows) >= 2 * rows * n * 4) == few
+
+
+@pytest.mark.parametrize("n,k,rows,few", [
+    # measured, 32-row tiles -> few-row kernel (us): 47 -> 58, 52 -> 65, 44 -> 51, 55 -> 64
+    (22532, 11008, 15, False), (31828, 8704, 23, False), (20716, 10752, 21, False), (32512, 9728, 17, False),
+    # 0.86 of the tiles' time
+    (4096, 14336, 12, True), (14336, 4096, 12, True), (14336, 8192, 16, True)])
+def test_few_row_kernel_below_half_the_cus(rq, n, k, rows, few):
+    """Q4_K where both kernels split K: the few-row kernel's ranges (at most 8 super-blocks, 4 above 16 rows) are not
+    to make more than two workgroups a CU; the tiles' plan is the policy's."""
+    w = _shape(rq, Q4K, n, k)
+    p, q = rq.gemm_policy(Q4K, k, n, rows), _plan_policy(rq, w, rows)
+    longest = 8 if rows <= 16 else 4
+    assert ((n + 255) // 256 * -(-k // 256 // longest) <= 512) == few
+    assert few or (p["splits"], p["sb_per_split"]) == (q.splits, q.sb_per_split)
+    assert not few or q.sb_per_split <= longest
 
 
 @pytest.mark.parametrize("ty,n,k,rows,n128", [
